@@ -205,16 +205,18 @@ int mrb_advance_timed(mrb_level *lvl, int nsteps, void *stream, double *kernel_m
  *   4  the two-pass step on 64x2-cell blocks;
  *   5  scaled FP16 storage only, no PRESSURE faces: the collide pass in
  *      FP32 arithmetic (FP64 sums of rho, E and the equilibria; the mass
- *      and energy residuals go to the rest direction);
+ *      and energy residuals go to the rest direction), on the tiles of 7;
  *   6  the two-pass step on 128x2-cell blocks;
- *   7  the two-pass step on 256x1-cell blocks;
- *   8  variant 5 on 256x1-cell blocks;
+ *   7  the two-pass step on tiles of 256 (shifted FP32: 128) consecutive
+ *      cells of a z-plane; FP64 levels of 2^18 cells and more run both
+ *      passes in one launch (mrb_advance_timed: its time in slot 0);
+ *   8  the same as 5;
  *   9  shifted FP32 storage only, no PRESSURE faces: the collide pass in
  *      FP32 arithmetic on the stored deviations from the rest state (FP64
  *      moments and equilibrium coefficients; mass and energy residuals on
  *      the rest direction, momentum residuals on the axis pairs),
  *      64x2-cell blocks;
- *  10  variant 9 on 256x1-cell blocks;
+ *  10  variant 9 on the tiles of 7;
  *  11  k_sweep: FP64 or shifted FP32 storage with rows of at most 256
  *      cells, one pass as a z-sweep with one resident block per x-row
  *      (MRB_E_UNSUPPORTED when the kernel's occupancy does not let every
@@ -227,7 +229,7 @@ int mrb_advance_timed(mrb_level *lvl, int nsteps, void *stream, double *kernel_m
  *  14+ the single-pass LDS z-sweep with different tile shapes.
  * The FP64-arithmetic variants give the same populations bit for bit; 5
  * and 8 give the same as each other, and 9, 10 and 13.  A level
- * starts on variant 7 (FP64 storage), 9 (shifted FP32) or 5 (scaled FP16).
+ * starts on variant 7 (FP64 storage), 10 (shifted FP32) or 5 (scaled FP16).
  * While a level has a PRESSURE face, variants 5 and 9 are replaced by 0 and
  * 4, 8 and 10 by 7, 13 by 11 (mrb_set_bc), and restored when the faces
  * change back.

@@ -292,6 +292,10 @@ struct mrb_level {
     // the launch count its tags start from
     uint64_t *d_sweep_qt = nullptr;
     uint32_t *d_sweep_epoch = nullptr;
+    // both passes in one launch (mrb_step.hip): work-list entries taken so
+    // far, and per tile the launch its Q_corr belongs to
+    unsigned long long *d_step_counter = nullptr;
+    uint32_t *d_step_flags = nullptr;
     // two-level link, held by the fine level (mrb_amr_link)
     mrb_level *amr_crse = nullptr;
     void *d_coal = nullptr;  // mrb::CoalesceEntry[n_coal]
@@ -381,12 +385,12 @@ constexpr int kNumTwoPassVariants = 14;
 constexpr int kOnePassVariant = 2;
 constexpr int kRows8Variant = 3;  // two passes on 64x8 blocks
 constexpr int kRows2Variant = 4;  // two passes on 64x2 blocks
-constexpr int kHalf32Variant = 5; // scaled FP16 storage, FP32 arithmetic in pass 2
+constexpr int kHalf32Variant = 5; // scaled FP16 storage, FP32 arithmetic in pass 2, tiles of consecutive cells
 constexpr int kX128Variant = 6;   // two passes on 128x2 blocks
-constexpr int kX256Variant = 7;   // two passes on 256x1 blocks
-constexpr int kHalf32X256Variant = 8; // variant 5 on 256x1 blocks
+constexpr int kX256Variant = 7;   // two passes on tiles of consecutive cells (mrb_step.hip)
+constexpr int kHalf32X256Variant = 8; // the same as 5
 constexpr int kF32Variant = 9;         // shifted FP32 storage, FP32 arithmetic in pass 2 (64x2 blocks)
-constexpr int kF32X256Variant = 10;    // variant 9 on 256x1 blocks
+constexpr int kF32X256Variant = 10;    // variant 9 on tiles of consecutive cells
 constexpr int kSweepVariant = 11;      // single-pass z-sweep, one block per x-row (FP64 / FP32, rows <= 256 cells)
 constexpr int kSweepRingPlanes = 8;    // planes of Q_y the z-sweep keeps for the rows beside
 constexpr int kSweepX64Variant = 12;   // the z-sweep on single-wave blocks of 64 cells of a row (FP64)
@@ -413,6 +417,16 @@ constexpr unsigned kConservationBlocks = 4096;
 unsigned conservation_blocks(const mrb_level *L);
 int conservation_partials(const mrb_level *L, double *part, hipStream_t s);
 int compact_two_pass_launch(mrb_level *L, int variant, hipStream_t s);
+// the two-pass step on 256-cell tiles of a z-plane (mrb_step.hip); reads the
+// current buffers, writes the spare ones, does not flip; ev (if not null)
+// receives events before, between and after the passes
+int compact_tile_step(mrb_level *L, bool fp32_collide, hipStream_t s, hipEvent_t *ev);
+// (32-bit byte offsets within a plane)
+inline bool tile_step_fits(const mrb_level *L) { return int64_t(L->ncell[0]) * L->ncell[1] < (int64_t(1) << 28); }
+inline uint32_t tiles_per_plane(int nx, int ny, int tile)
+{
+    return (uint32_t(nx) * uint32_t(ny) + uint32_t(tile) - 1u) / uint32_t(tile);
+}
 int compact_variant_launch(mrb_level *L, int index, hipStream_t s);
 const char *compact_variant_name(int index);
 // FillBoundary of one lattice's current fab buffer (mrb_level.hip)

@@ -1066,13 +1066,13 @@ int mrb_level_create(const mrb_level_desc *desc, mrb_level **out)
     L->layout = desc->layout;
     L->nlattice = desc->nlattice;
     L->storage = desc->storage;
-    // the default step variant per storage: two passes on 256x1-cell blocks
-    // for FP64; for the reduced storages the FP32-arithmetic collide (64x2
-    // blocks for shifted FP32, 64x4 for scaled FP16), which levels with
-    // PRESSURE faces replace by FP64 arithmetic (mrb_set_bc);
+    // the default step variant per storage: two passes on tiles of
+    // consecutive cells; for the reduced storages with the FP32-arithmetic
+    // collide, which levels with PRESSURE faces replace by FP64 arithmetic
+    // (mrb_set_bc);
     // mrb_set_hot_kernel and mrb_autotune select others
     L->hot = L->storage == MRB_STORAGE_F64            ? kX256Variant
-             : L->storage == MRB_STORAGE_F32_SHIFTED ? kF32Variant
+             : L->storage == MRB_STORAGE_F32_SHIFTED ? kF32X256Variant
                                                       : kHalf32Variant;
     L->hot_default = true;
     L->hot_h32 = -1;
@@ -1208,6 +1208,11 @@ int mrb_level_create(const mrb_level_desc *desc, mrb_level **out)
         MRB_HIP(hipMemset(L->d_mask, 0, sizeof(uint32_t) * T));
         MRB_HIP(hipMalloc(&L->d_q, sizeof(double) * 3 * T));
         MRB_HIP(hipMemset(L->d_q, 0, sizeof(double) * 3 * T));
+        const size_t ntiles = size_t(tiles_per_plane(L->ncell[0], L->ncell[1], 256)) * size_t(L->ncell[2]);
+        MRB_HIP(hipMalloc(&L->d_step_counter, sizeof(unsigned long long)));
+        MRB_HIP(hipMemset(L->d_step_counter, 0, sizeof(unsigned long long)));
+        MRB_HIP(hipMalloc(&L->d_step_flags, sizeof(uint32_t) * ntiles));
+        MRB_HIP(hipMemset(L->d_step_flags, 0, sizeof(uint32_t) * ntiles));
         if (L->storage == MRB_STORAGE_F64 || L->storage == MRB_STORAGE_F32_SHIFTED) {
             const size_t plane = size_t(L->ncell[0]) * size_t(L->ncell[1]);
             const size_t nblk = size_t((L->ncell[0] + 63) / 64) * size_t(L->ncell[1]);
@@ -1270,6 +1275,8 @@ int mrb_level_destroy(mrb_level *L)
     (void)hipFree(L->d_md);
     (void)hipFree(L->d_dq);
     (void)hipFree(L->d_q);
+    (void)hipFree(L->d_step_counter);
+    (void)hipFree(L->d_step_flags);
     (void)hipFree(L->d_red);
     (void)hipFree(L->d_small);
     for (auto &e : L->ev)
