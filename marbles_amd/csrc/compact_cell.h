@@ -518,8 +518,6 @@ __device__ __forceinline__ PullBits pull_settle(const T *__restrict__ f, const C
         if (__any(S.nondirect(mask) != 0u))
             pb = pull_raw<BCX, T, false, NT>(f, A, x, y, z, cell, mask, rf, rg);
     }
-    // (one continuation for every path)
-    asm volatile("" : "+v"(pb.cmask));
     return pb;
 }
 

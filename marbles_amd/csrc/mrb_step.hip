@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(kStepTile, 2) k_step(
 
 // the passes apart
 template <class T, int BCX, int TILE>
-__global__ void __launch_bounds__(TILE, 2) k_qpass_tile(
+__global__ void __launch_bounds__(TILE) k_qpass_tile(
     const T *__restrict__ f, const uint32_t *__restrict__ mask, double *__restrict__ Q, CompactArgs A, BCDev bc,
     ShiftTab sh, Half16 h16, CollideParams P, TileArgs G)
 {
