@@ -66,19 +66,10 @@ __global__ void __launch_bounds__(kAmrBlock) k_coalesce(
 // (k_explode): ((c + o_x s_x) + o_y s_y) + o_z s_z with o = -+1/4.
 // Every load is issued unconditionally: the fab's ghost layers (ng >= 2,
 // checked when the map is built) hold P +- 2 in every direction.
-__global__ void __launch_bounds__(kAmrBlock) k_explode_slopes(
-    const double *__restrict__ crse, const BoxDev *__restrict__ cboxes, const ExplodeParent *__restrict__ par,
-    int64_t npar, double *__restrict__ out)
+// the coarse value and the limited slopes of one component of the parent at c
+__device__ __forceinline__ void parent_slopes(const double *__restrict__ c, const BoxDev &CB, int fl, double out[4])
 {
-    const int64_t t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= npar * NQ) return;
-    const int q = int(t / npar);
-    const int64_t p = t - int64_t(q) * npar;
-    const ExplodeParent P = par[p];
-    const BoxDev &CB = cboxes[P.crse_box];
-    const double *c = crse + CB.base * NQ + int64_t(q) * CB.ncell + P.crse_local;
     const int64_t st[3] = {1, CB.n[0], int64_t(CB.n[0]) * CB.n[1]};
-    const int fl = P.flags;
     double u[27];
     for (int oz = -1; oz <= 1; ++oz)
         for (int oy = -1; oy <= 1; ++oy)
@@ -127,8 +118,56 @@ __global__ void __launch_bounds__(kAmrBlock) k_explode_slopes(
         if (dumax * alpha > (umax - uc)) alpha = (umax - uc) / dumax;
         if (dumax * alpha > (uc - umin)) alpha = (uc - umin) / dumax;
     }
-    out[(int64_t(0) * NQ + q) * npar + p] = uc;
-    for (int d = 0; d < 3; ++d) out[(int64_t(1 + d) * NQ + q) * npar + p] = s[d] * alpha;
+    out[0] = uc;
+    for (int d = 0; d < 3; ++d) out[1 + d] = s[d] * alpha;
+}
+
+__global__ void __launch_bounds__(kAmrBlock) k_explode_slopes(
+    const double *__restrict__ crse, const BoxDev *__restrict__ cboxes, const ExplodeParent *__restrict__ par,
+    int64_t npar, double *__restrict__ out)
+{
+    const int64_t t = xcd_block() * blockDim.x + threadIdx.x;
+    if (t >= npar * NQ) return;
+    const int q = int(t / npar);
+    const int64_t p = t - int64_t(q) * npar;
+    const ExplodeParent P = par[p];
+    const BoxDev &CB = cboxes[P.crse_box];
+    double v[4];
+    parent_slopes(crse + CB.base * NQ + int64_t(q) * CB.ncell + P.crse_local, CB, P.flags, v);
+    for (int k = 0; k < 4; ++k) out[(int64_t(k) * NQ + q) * npar + p] = v[k];
+}
+
+// The two-level step's explosion, both lattices (blockIdx.z) and one
+// component per blockIdx.y: a thread forms the slopes of one coarse parent
+// and writes the children that are ghosts of one fine box (listed in the
+// order of the fab, so that neighbouring threads read and write neighbouring
+// cells).  Through an array of slopes, written per parent and read back by
+// every child, the pair of lattices took 728 of 5640 us of a coarse step at
+// 128x128x64.
+__global__ void __launch_bounds__(kAmrBlock) k_explode_groups(
+    const double *__restrict__ crse_f, const double *__restrict__ crse_g, double *__restrict__ fine_f,
+    double *__restrict__ fine_g, const BoxDev *__restrict__ cboxes, const BoxDev *__restrict__ fboxes,
+    const ExplodeGroup *__restrict__ groups, int64_t n)
+{
+    const int64_t t = int64_t(xcd_index(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const int q = int(blockIdx.y);
+    const double *crse = blockIdx.z ? crse_g : crse_f;
+    double *fine = blockIdx.z ? fine_g : fine_f;
+    const ExplodeGroup G = groups[t];
+    const BoxDev &CB = cboxes[G.crse_box];
+    const BoxDev &FB = fboxes[G.fine_box];
+    double v[4];
+    parent_slopes(crse + CB.base * NQ + int64_t(q) * CB.ncell + G.crse_local, CB, G.flags, v);
+    double *fo = fine + FB.base * NQ + int64_t(q) * FB.ncell + G.fine_local;
+    const int64_t sy = FB.n[0], sz = int64_t(FB.n[0]) * FB.n[1];
+    for (int ch = 0; ch < 8; ++ch) {
+        if (!((G.children >> ch) & 1)) continue;
+        const double ox = (ch & 1) ? 0.25 : -0.25;
+        const double oy = (ch & 2) ? 0.25 : -0.25;
+        const double oz = (ch & 4) ? 0.25 : -0.25;
+        fo[(ch & 1) + ((ch >> 1) & 1) * sy + (ch >> 2) * sz] = v[0] + ox * v[1] + oy * v[2] + oz * v[3];
+    }
 }
 
 __global__ void __launch_bounds__(kAmrBlock) k_explode(
@@ -326,11 +365,9 @@ void amr_release(mrb_level *L)
     L->cap_stream = nullptr;
     if (L->d_coal) (void)hipFree(L->d_coal);
     if (L->d_expl) (void)hipFree(L->d_expl);
-    if (L->d_expl_par) (void)hipFree(L->d_expl_par);
-    if (L->d_expl_slopes) (void)hipFree(L->d_expl_slopes);
-    L->d_expl_par = nullptr;
-    L->d_expl_slopes = nullptr;
-    L->n_expl_par = 0;
+    if (L->d_expl_groups) (void)hipFree(L->d_expl_groups);
+    L->d_expl_groups = nullptr;
+    L->n_expl_groups = 0;
     L->expl_crse_depth = 1;
     if (L->d_coal_cell) (void)hipFree(L->d_coal_cell);
     if (L->d_coal_vals) (void)hipFree(L->d_coal_vals);
@@ -475,6 +512,52 @@ int mrb_amr_link(mrb_level *crse, mrb_level *fine)
         if (ring[o] == 1) qring.push_back(expl[o]);
     }
     expl.swap(sorted);
+    // the explosion's groups: one per (fine box, parent) with the children
+    // that are uncovered ghosts of the box, in the order of the box's fab
+    std::vector<ExplodeGroup> groups;
+    {
+        std::vector<std::pair<std::pair<int32_t, int64_t>, uint32_t>> gk;  // (box, child (0,0,0)), entry
+        gk.reserve(expl.size());
+        for (size_t n = 0; n < expl.size(); ++n) {
+            const BoxDev &FB = fine->boxes[expl[n].fine_box];
+            const int b = expl[n].bits & 7;
+            const int64_t l0 = expl[n].fine_local - (b & 1) - ((b >> 1) & 1) * int64_t(FB.n[0]) -
+                               (b >> 2) * int64_t(FB.n[0]) * FB.n[1];
+            gk.push_back({{expl[n].fine_box, l0}, uint32_t(n)});
+        }
+        std::sort(gk.begin(), gk.end());
+        for (const auto &g : gk) {
+            const ExplodeEntry &e = expl[g.second];
+            if (groups.empty() || groups.back().fine_box != g.first.first ||
+                groups.back().fine_local != g.first.second) {
+                ExplodeGroup G{};
+                G.fine_local = g.first.second;
+                G.fine_box = e.fine_box;
+                G.crse_local = e.crse_local;
+                G.crse_box = e.crse_box;
+                G.flags = parents.list[size_t(e.parent)].flags;
+                groups.push_back(G);
+            }
+            groups.back().children |= 1 << (e.bits & 7);
+        }
+    }
+    // With 3 ghost layers a ring-3 cell's streamed population that a ring-2
+    // cell pulls in the next substep comes from beyond the fab: the -1
+    // sentinel.  Such sources are marked in the entry (bit 3 + q) and read as
+    // -1, and the first substep streams rings 1 and 2 only.
+    if (fine->ng == 3) {
+        std::vector<uint8_t> ring3(size_t(fine->total_cells), 0);
+        for (const ExplodeEntry &e : expl)
+            if (ring_of(e) == 3) ring3[size_t(fine->boxes[e.fine_box].base + e.fine_local)] = 1;
+        for (ExplodeEntry &e : expl) {
+            const BoxDev &FB = fine->boxes[e.fine_box];
+            const int64_t sy = FB.n[0], sz = int64_t(FB.n[0]) * FB.n[1];
+            if (ring_of(e) > 2) continue;  // (a ring-2 cell's sources lie in the fab)
+            for (int q = 1; q < NQ; ++q)
+                if (ring3[size_t(FB.base + e.fine_local - (kEV[q][0] + kEV[q][1] * sy + kEV[q][2] * sz))])
+                    e.bits |= 1 << (3 + q);
+        }
+    }
     // The fine level's FillBoundary inside the two-level step: every first-
     // layer ghost (the pulls of valid cells), and deeper ghosts only where
     // a kernel of the step reads them: next to an uncovered ghost (the
@@ -547,13 +630,12 @@ int mrb_amr_link(mrb_level *crse, mrb_level *fine)
     }
     if ((rc = check_parents(crse, parents))) return rc;
     amr_release(fine);
-    if (!parents.list.empty()) {
-        MRB_HIP(hipMalloc(&fine->d_expl_par, sizeof(ExplodeParent) * parents.list.size()));
-        MRB_HIP(hipMemcpy(fine->d_expl_par, parents.list.data(), sizeof(ExplodeParent) * parents.list.size(),
+    if (!groups.empty()) {
+        MRB_HIP(hipMalloc(&fine->d_expl_groups, sizeof(ExplodeGroup) * groups.size()));
+        MRB_HIP(hipMemcpy(fine->d_expl_groups, groups.data(), sizeof(ExplodeGroup) * groups.size(),
                           hipMemcpyHostToDevice));
-        MRB_HIP(hipMalloc(&fine->d_expl_slopes, sizeof(double) * 4 * NQ * parents.list.size()));
     }
-    fine->n_expl_par = int64_t(parents.list.size());
+    fine->n_expl_groups = int64_t(groups.size());
     fine->expl_crse_depth = parents.depth;
     if (!coal.empty()) {
         MRB_HIP(hipMalloc(&fine->d_coal, sizeof(CoalesceEntry) * coal.size()));
@@ -606,10 +688,43 @@ int mrb_coalesce(const mrb_level *fine, mrb_level *crse, void *stream)
 }
 
 namespace mrb {
-// the two-level fillpatch of one lattice; `step_map`: the fine FillBoundary
-// covers what the two-level step reads (the linked pair's step map) rather
-// than every ghost layer
-static int explode_impl(const mrb_level *crse, mrb_level *fine, int lattice, hipStream_t s, bool step_map);
+// fine ghosts over uncovered domain from the coarse level, lattices
+// first .. first + count - 1, then the boundary functor
+static int explode_uncovered(const mrb_level *crse, mrb_level *fine, int first, int count, hipStream_t s)
+{
+    if (fine->n_expl_groups > 0) {
+        const int last = first + count - 1;
+        k_explode_groups<<<dim3(blocks_for(fine->n_expl_groups), NQ, unsigned(count)), kAmrBlock, 0, s>>>(
+            (const double *)crse->pop[first][crse->cur], (const double *)crse->pop[last][crse->cur],
+            (double *)fine->pop[first][fine->cur], (double *)fine->pop[last][fine->cur], crse->d_boxes, fine->d_boxes,
+            (const ExplodeGroup *)fine->d_expl_groups, fine->n_expl_groups);
+        MRB_HIP(hipGetLastError());
+    }
+    for (int l = first; l < first + count; ++l) {
+        const int rc = mrb_physbc(fine, l, s);
+        if (rc) return rc;
+    }
+    return MRB_OK;
+}
+// the slopes read the coarse parents' neighbourhoods: FillBoundary of the
+// coarse level (ghost layers only, so its valid data is unchanged)
+static int explode_coarse_ghosts(const mrb_level *crse, const mrb_level *fine, hipStream_t s)
+{
+    const int depth = std::max(1, fine->expl_crse_depth);
+    if (crse->fresh_depth >= depth) return MRB_OK;
+    return fab_fill_boundary_depth(const_cast<mrb_level *>(crse), depth, s);
+}
+// the fine FillBoundary of the two-level step, both lattices: what the step
+// reads (the linked pair's step map) rather than every ghost layer
+static int fill_fine_step(mrb_level *fine, hipStream_t s)
+{
+    const bool part = fine->d_gmap_step != nullptr;
+    const int rc = part ? fab_fill_boundary_map(fine, fine->d_gmap_step, fine->n_gmap_step, s)
+                        : fab_fill_boundary_depth(fine, fine->ng, s);
+    if (rc) return rc;
+    fine->fresh_depth = part ? 1 : fine->ng;
+    return MRB_OK;
+}
 }  // namespace mrb
 
 int mrb_explode(const mrb_level *crse, mrb_level *fine, int lattice, void *stream)
@@ -617,40 +732,16 @@ int mrb_explode(const mrb_level *crse, mrb_level *fine, int lattice, void *strea
     if (!fine || !crse) return set_error(MRB_E_ARG, "null level");
     if (fine->amr_crse != crse) return set_error(MRB_E_STATE, "levels are not linked (mrb_amr_link)");
     if (lattice < 0 || lattice > 1) return set_error(MRB_E_ARG, "lattice must be 0 or 1");
-    return explode_impl(crse, fine, lattice, as_stream(stream), false);
-}
-
-namespace mrb {
-static int explode_impl(const mrb_level *crse, mrb_level *fine, int lattice, hipStream_t s, bool step_map)
-{
-    // the slopes read the coarse parents' neighbourhoods: FillBoundary of
-    // the coarse level (ghost layers only, so its valid data is unchanged)
-    const int depth = std::max(1, fine->expl_crse_depth);
-    int rc;
-    if (crse->fresh_depth < depth &&
-        (rc = fab_fill_boundary_depth(const_cast<mrb_level *>(crse), depth, s)))
-        return rc;
+    hipStream_t s = as_stream(stream);
     // fine-fine ghosts first, then the uncovered ones, then the domain
     // boundary (the three sets of cells are disjoint; physbc reads valid
     // and in-domain ghost cells only)
-    const bool part = step_map && fine->d_gmap_step;
-    rc = part ? fab_fill_boundary_map(fine, lattice, fine->d_gmap_step, fine->n_gmap_step, s)
-              : fab_fill_boundary(fine, lattice, s);
+    int rc = explode_coarse_ghosts(crse, fine, s);
+    if (!rc) rc = fab_fill_boundary(fine, lattice, s);
     if (rc) return rc;
-    if (lattice == 1) fine->fresh_depth = part ? 1 : fine->ng;
-    if (fine->n_expl > 0) {
-        k_explode_slopes<<<blocks_for(fine->n_expl_par * NQ), kAmrBlock, 0, s>>>(
-            (const double *)crse->pop[lattice][crse->cur], crse->d_boxes, (const ExplodeParent *)fine->d_expl_par,
-            fine->n_expl_par, fine->d_expl_slopes);
-        MRB_HIP(hipGetLastError());
-        k_explode<<<blocks_for(fine->n_expl), kAmrBlock, 0, s>>>(
-            fine->d_expl_slopes, fine->n_expl_par, (double *)fine->pop[lattice][fine->cur], fine->d_boxes,
-            (const ExplodeEntry *)fine->d_expl, fine->n_expl);
-        MRB_HIP(hipGetLastError());
-    }
-    return mrb_physbc(fine, lattice, s);
+    if (lattice == 1) fine->fresh_depth = fine->ng;
+    return explode_uncovered(crse, fine, lattice, 1, s);
 }
-}  // namespace mrb
 
 static int check_advance(mrb_level *crse, mrb_level *fine)
 {
@@ -677,26 +768,20 @@ static int amr_step(mrb_level *crse, mrb_level *fine, void *stream)
     if (crse->fresh_depth < depth && (rc = fab_fill_boundary_depth(crse, depth, s))) return rc;
     for (int l = 0; l < 2; ++l)
         if ((rc = mrb_physbc(crse, l, stream))) return rc;
-    for (int l = 0; l < 2; ++l)
-        if ((rc = explode_impl(crse, fine, l, s, true))) return rc;
+    if ((rc = explode_coarse_ghosts(crse, fine, s))) return rc;
+    if ((rc = fill_fine_step(fine, s))) return rc;
+    if ((rc = explode_uncovered(crse, fine, 0, 2, s))) return rc;
     for (int sub = 0; sub < 2; ++sub) {
         for (int l = 0; l < 2; ++l)
             if ((rc = mrb_physbc(fine, l, stream))) return rc;
         // time_step(1) -> advance(1) (LBM.cpp:523-544): stream f, g and
         // collide as one batched step
-        fine->stream_rings_le2 = sub == 1;
+        fine->stream_substep = sub + 1;
         rc = fab_batched_step(fine, nullptr, 0, s);
-        fine->stream_rings_le2 = false;
+        fine->stream_substep = 0;
         if (rc) return rc;
-        if (sub == 0) {
-            // the ghosts the second substep reads
-            for (int l = 0; l < 2; ++l) {
-                rc = fine->d_gmap_step ? fab_fill_boundary_map(fine, l, fine->d_gmap_step, fine->n_gmap_step, s)
-                                       : fab_fill_boundary(fine, l, s);
-                if (rc) return rc;
-            }
-            fine->fresh_depth = fine->d_gmap_step ? 1 : fine->ng;
-        }
+        // the ghosts the second substep reads
+        if (sub == 0 && (rc = fill_fine_step(fine, s))) return rc;
     }
     // advance(0): stream, average_down_to, collide, with the coalescence
     // fused into the coarse passes

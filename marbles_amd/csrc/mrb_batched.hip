@@ -12,7 +12,7 @@
 // streamed state.  The Q of a ring-1 ghost cell comes from its owning box
 // by FillBoundary, as the reference's macrodata does (LBM.cpp:905); on a
 // fine level the ring-1 ghost cells over uncovered domain have no owner
-// and compute Q from their own pulled populations (k_fab_qpass_listed).
+// and compute Q from their own streamed populations (k_stream_listed).
 // Those uncovered ghost cells also keep the streamed values that the
 // reference keeps (they feed the second substep and the coalescence), so
 // they are streamed from the explosion map; all other ghost values are
@@ -187,31 +187,6 @@ __global__ void __launch_bounds__(kFabTile) k_fab_qpass(
     }
 }
 
-// pass 1 at the listed ghost cells (the first n entries of the explosion
-// map, which are the ring-1 cells)
-__global__ void __launch_bounds__(256) k_fab_qpass_listed(
-    const double *__restrict__ f, const double *__restrict__ g, double *__restrict__ Q,
-    const BoxDev *__restrict__ boxes, const uint32_t *__restrict__ mask, const ExplodeEntry *__restrict__ list,
-    int64_t n, CollideParams P)
-{
-    const int64_t t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const ExplodeEntry e = list[t];
-    const BoxDev &B = boxes[e.fine_box];
-    const int64_t loc = e.fine_local;
-    const uint32_t m = mask[B.base + loc];
-    if (!(m & 1u)) return;
-    double fv[NQ], gv[NQ];
-    pull_fab(f, g, B, loc, m, fv, gv);
-    double rho, jx, jy, jz, E;
-    accumulate_q_moments(fv, gv, rho, jx, jy, jz, E);
-    const Macro M = macro_from(rho, jx, jy, jz, E, P);
-    double *q = Q + B.base * 3 + loc;
-    q[0] = M.Qx;
-    q[B.ncell] = M.Qy;
-    q[2 * B.ncell] = M.Qz;
-}
-
 template <bool COAL>
 __global__ void __launch_bounds__(kFabTile) k_fab_collide(
     const double *__restrict__ f, const double *__restrict__ g, double *__restrict__ fo,
@@ -268,15 +243,23 @@ __global__ void __launch_bounds__(kFabTile) k_fab_collide(
 }
 
 // LBM::stream (LBM.cpp:558-604) at the listed ghost cells (fine cells over
-// uncovered domain, from the explosion map): pull with the in-fab test
+// uncovered domain, from the explosion map): pull with the in-fab test.  A
+// ring-1 cell's streamed values are the post-stream state whose Q_corr pass 1
+// would form there, so it is formed here from the same registers (a pass of
+// its own over the ring-1 cells pulled their 54 populations again: 292 of
+// 5640 us of a coarse step at 128x128x64).
 __global__ void __launch_bounds__(256) k_stream_listed(
     const double *__restrict__ f, const double *__restrict__ g, double *__restrict__ fo,
-    double *__restrict__ go, const uint32_t *__restrict__ mask, const BoxDev *__restrict__ boxes,
-    const ExplodeEntry *__restrict__ list, int64_t n)
+    double *__restrict__ go, double *__restrict__ Q, const uint32_t *__restrict__ mask,
+    const BoxDev *__restrict__ boxes, const ExplodeEntry *__restrict__ list, int64_t n, int ring3_minus1,
+    CollideParams P)
 {
     const int64_t t = xcd_block() * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const ExplodeEntry e = list[t];
+    // second substep: directions whose source is an uncovered ring-3 ghost,
+    // which holds the -1 sentinel there (mrb_amr_link)
+    const uint32_t minus = ring3_minus1 ? uint32_t(e.bits) >> 3 : 0u;
     const BoxDev &B = boxes[e.fine_box];
     const int64_t loc = e.fine_local;
     const int64_t nxy = int64_t(B.n[0]) * B.n[1];
@@ -307,7 +290,7 @@ __global__ void __launch_bounds__(256) k_stream_listed(
                                    : int64_t(kBounce[q]) * B.ncell + loc;
         vf[q] = fb[idx];
         vg[q] = gb[idx];
-        keep |= uint32_t(use) << q;
+        keep |= uint32_t(use && !(direct && ((minus >> q) & 1u))) << q;
     });
     static_for<NQ>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -315,6 +298,18 @@ __global__ void __launch_bounds__(256) k_stream_listed(
         fob[q * B.ncell + loc] = use ? vf[q] : -1.0;
         gob[q * B.ncell + loc] = use ? vg[q] : -1.0;
     });
+    // ring 1: next to the valid box (its sources all lie in the fab)
+    const int i = ii + B.lo[0], j = jj + B.lo[1], k = kk + B.lo[2];
+    if (fluid && i >= B.vlo[0] - 1 && i <= B.vhi[0] + 1 && j >= B.vlo[1] - 1 && j <= B.vhi[1] + 1 &&
+        k >= B.vlo[2] - 1 && k <= B.vhi[2] + 1) {
+        double rho, jx, jy, jz, E;
+        accumulate_q_moments(vf, vg, rho, jx, jy, jz, E);
+        const Macro M = macro_from(rho, jx, jy, jz, E, P);
+        double *q = Q + B.base * 3 + loc;
+        q[0] = M.Qx;
+        q[B.ncell] = M.Qy;
+        q[2 * B.ncell] = M.Qz;
+    }
 }
 
 // per fab cell: bit q = is_fluid(x - c_q) != 0 (sources inside the fab),
@@ -538,9 +533,14 @@ int fab_batched_passes(mrb_level *L, const mrb_level *coal_from, hipStream_t s)
     else
         k_fab_qpass<false><<<gc, kFabTile, 0, s>>>(f, g, L->d_dq, L->d_tiles_c, A, C, L->cp);
     MRB_HIP(hipGetLastError());
-    if (L->n_qring > 0) {
-        k_fab_qpass_listed<<<unsigned((L->n_qring + 255) / 256), 256, 0, s>>>(
-            f, g, L->d_dq, L->d_boxes, L->d_mask, (const ExplodeEntry *)L->d_qring, L->n_qring, L->cp);
+    // the listed ghosts stream before pass 2, which reads their Q_corr
+    // (the two-level step: what the second substep and the coalescence read)
+    const bool rings12 = L->stream_substep == 2 || (L->stream_substep == 1 && L->ng == 3);
+    const int64_t nst = rings12 ? L->n_expl_le2 : L->n_expl;
+    if (nst > 0) {
+        k_stream_listed<<<unsigned((nst + 255) / 256), 256, 0, s>>>(
+            f, g, fo, go, L->d_dq, L->d_mask, L->d_boxes, (const ExplodeEntry *)L->d_expl, nst,
+            L->stream_substep == 2 && L->ng == 3, L->cp);
         MRB_HIP(hipGetLastError());
     }
     int rc = fab_fill_boundary_q(L, s);
@@ -550,12 +550,6 @@ int fab_batched_passes(mrb_level *L, const mrb_level *coal_from, hipStream_t s)
     else
         k_fab_collide<false><<<gc, kFabTile, 0, s>>>(f, g, fo, go, L->d_dq, L->d_tiles_c, A, C, L->cp);
     MRB_HIP(hipGetLastError());
-    const int64_t nst = L->stream_rings_le2 ? L->n_expl_le2 : L->n_expl;
-    if (nst > 0) {
-        k_stream_listed<<<unsigned((nst + 255) / 256), 256, 0, s>>>(
-            f, g, fo, go, L->d_mask, L->d_boxes, (const ExplodeEntry *)L->d_expl, nst);
-        MRB_HIP(hipGetLastError());
-    }
     return MRB_OK;
 }
 

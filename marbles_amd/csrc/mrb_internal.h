@@ -113,7 +113,8 @@ struct ExplodeEntry {
     int64_t crse_local;  // the parent
     int32_t fine_box;
     int32_t crse_box;
-    int32_t bits;    // bit d: high child in direction d
+    int32_t bits;    // bit d: high child in direction d; bit 3 + q: the source
+                     // x - c_q is an uncovered ring-3 ghost (mrb_amr_link)
     int32_t parent;  // index of the parent in the level's ExplodeParent list
 };
 
@@ -127,6 +128,15 @@ struct ExplodeParent {
     int64_t crse_local;
     int32_t crse_box;
     int32_t flags;
+};
+
+// the children of one coarse parent that are uncovered ghosts of one fine
+// box: fine_local = child (0, 0, 0) in the box's fab (possibly outside it),
+// children = a bit per child (x fastest), the rest as ExplodeParent
+struct ExplodeGroup {
+    int64_t crse_local, fine_local;
+    int32_t crse_box, fine_box;
+    int32_t flags, children;
 };
 
 // Single-pass z-sweep kernel shapes: rows per tile and z planes per chunk.
@@ -302,9 +312,8 @@ struct mrb_level {
     int64_t n_coal = 0;
     void *d_expl = nullptr;  // mrb::ExplodeEntry[n_expl]
     int64_t n_expl = 0;
-    void *d_expl_par = nullptr;  // mrb::ExplodeParent[n_expl_par]
-    int64_t n_expl_par = 0;
-    double *d_expl_slopes = nullptr;  // [4 * NQ][parent]: value and limited slopes of one lattice
+    void *d_expl_groups = nullptr;  // mrb::ExplodeGroup[n_expl_groups]
+    int64_t n_expl_groups = 0;
     int expl_crse_depth = 1;          // coarse FillBoundary depth the interpolation reads
     int32_t *d_coal_cell = nullptr;  // per coarse fab cell: coalescence entry or -1
     double *d_coal_vals = nullptr;   // [2q + lattice][entry]: masked means of the children
@@ -314,7 +323,7 @@ struct mrb_level {
     int64_t n_expl_le2 = 0;
     void *d_qring = nullptr;  // mrb::ExplodeEntry[n_qring]
     int64_t n_qring = 0;
-    bool stream_rings_le2 = false;  // the listed ghost stream covers rings 1-2 only
+    int stream_substep = 0;  // substep of the two-level step under way (0: none)
     // batched fab-layout step: tile list of the valid cells and the number
     // of persistent blocks (0 = one block per tile)
     mrb::FabTile *d_tiles_c = nullptr;
@@ -431,8 +440,8 @@ int compact_variant_launch(mrb_level *L, int index, hipStream_t s);
 const char *compact_variant_name(int index);
 // FillBoundary of one lattice's current fab buffer (mrb_level.hip)
 int fab_fill_boundary(mrb_level *L, int lattice, hipStream_t s);
-// FillBoundary of one lattice's current fab buffer over the given map
-int fab_fill_boundary_map(mrb_level *L, int lattice, const GhostPair *map, int64_t n, hipStream_t s);
+// FillBoundary of both lattices' current fab buffers over the given map
+int fab_fill_boundary_map(mrb_level *L, const GhostPair *map, int64_t n, hipStream_t s);
 // every ghost cell (within `depth` layers) that FillBoundary writes, with its owner
 void build_ghost_map(const mrb_level *L, int depth, std::vector<GhostPair> &map);
 // FillBoundary of both lattices, `depth` ghost layers (1 or ng); sets fresh_depth

@@ -55,13 +55,24 @@ __device__ __forceinline__ int find_box(const int64_t *__restrict__ base, int nb
     return lo;
 }
 
+// the same for the cells c = blockIdx.x * blockDim.x + threadIdx.x of a flat
+// launch: the search runs once per block on scalar values, from its first
+// cell, and each lane moves on to its own box
+__device__ __forceinline__ int find_box_flat(const int64_t *__restrict__ base, int nbox, int64_t c)
+{
+    int b = find_box(base, nbox, int64_t(blockIdx.x) * blockDim.x);
+    while (b + 1 < nbox && base[b + 1] <= c) ++b;
+    return b;
+}
+
+// (a fab holds fewer than 2^31 cells)
 __device__ __forceinline__ void local_to_ijk(const BoxDev &B, int64_t loc, int &i, int &j, int &k)
 {
-    const int64_t nxy = int64_t(B.n[0]) * B.n[1];
-    k = int(loc / nxy);
-    const int64_t r = loc - int64_t(k) * nxy;
-    j = int(r / B.n[0]);
-    i = int(r - int64_t(j) * B.n[0]);
+    const uint32_t nx = uint32_t(B.n[0]), nxy = nx * uint32_t(B.n[1]), l = uint32_t(loc);
+    k = int(l / nxy);
+    const uint32_t r = l - uint32_t(k) * nxy;
+    j = int(r / nx);
+    i = int(r - uint32_t(j) * nx);
     i += B.lo[0];
     j += B.lo[1];
     k += B.lo[2];
@@ -89,10 +100,13 @@ __device__ __forceinline__ int64_t loc_of(const BoxDev &B, int i, int j, int k)
 // ---------------------------------------------------------------------------
 template <class T, int NC>
 __global__ void k_fill_map(
-    T *__restrict__ arr, const BoxDev *__restrict__ boxes, const GhostPair *__restrict__ map, int64_t nmap)
+    T *__restrict__ arr, T *__restrict__ arr2, const BoxDev *__restrict__ boxes, const GhostPair *__restrict__ map,
+    int64_t nmap)
 {
+    // (blockIdx.y == 1: the second array, of the same shape)
     const int64_t t = xcd_block() * blockDim.x + threadIdx.x;
     if (t >= nmap) return;
+    if (blockIdx.y) arr = arr2;
     const GhostPair p = map[t];
     const int64_t dn = boxes[p.dst_box].ncell, sn = boxes[p.src_box].ncell;
     T *dst = arr + boxes[p.dst_box].base * NC + p.dst_local;
@@ -110,30 +124,38 @@ __global__ void k_fill_map(
 // which is exactly the value the reference's push leaves in its -1
 // pre-filled temporary (each (y,p) has at most one writer).
 // ---------------------------------------------------------------------------
-__global__ void k_stream_fab(
-    const double *__restrict__ fin, double *__restrict__ fout, const int32_t *__restrict__ isf,
+// mask: bit q = the source y - c_q is inside the fab and fluid, bit 0 = own
+// fluid.  Every load is issued (a value that is not used reads the cell
+// itself), the sentinel selected afterwards.
+__global__ void __launch_bounds__(kBlock) k_stream_fab(
+    const double *__restrict__ fin, double *__restrict__ fout, const uint32_t *__restrict__ mask,
     const BoxDev *__restrict__ boxes, const int64_t *__restrict__ base, int nbox, int64_t total)
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const uint32_t m = mask[c];
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int i, j, k;
     local_to_ijk(B, loc, i, j, k);
     const double *f = fin + B.base * NQ;
     double *fo = fout + B.base * NQ;
-    const int32_t *fl = isf + B.base * 2;
-    const bool fluid = fl[loc] == 1;
+    const int64_t sy = B.n[0], sz = int64_t(B.n[0]) * B.n[1];
+    const bool fluid = m & 1u;
+    double v[NQ];
+    uint32_t keep = 0;
     static_for<NQ>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        const int a = i - ev(q, 0), bb = j - ev(q, 1), e = k - ev(q, 2);
-        double v = -1.0;
-        if (fluid && in_fab(B, a, bb, e)) {
-            const int64_t sl = loc_of(B, a, bb, e);
-            v = fl[sl] != 0 ? f[q * B.ncell + sl] : f[kBounce[q] * B.ncell + loc];
-        }
-        fo[q * B.ncell + loc] = v;
+        constexpr int cx = ev(q, 0), cy = ev(q, 1), cz = ev(q, 2);
+        const bool use = fluid && in_fab(B, i - cx, j - cy, k - cz);
+        const bool direct = use && ((m >> q) & 1u);
+        v[q] = f[direct ? int64_t(q) * B.ncell + loc - (cx + cy * sy + cz * sz) : int64_t(kBounce[q]) * B.ncell + loc];
+        keep |= uint32_t(use) << q;
+    });
+    static_for<NQ>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        fo[q * B.ncell + loc] = ((keep >> q) & 1u) ? v[q] : -1.0;
     });
 }
 
@@ -249,7 +271,7 @@ __global__ void k_moments_fab(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int i, j, k;
@@ -301,7 +323,7 @@ __global__ void k_dq_fab(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int iv[3];
@@ -363,7 +385,7 @@ __global__ void k_plot_derived_fab(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int iv[3];
@@ -402,7 +424,7 @@ __global__ void k_eqrelax_fab(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int i, j, k;
@@ -489,7 +511,7 @@ __global__ void k_flags_body(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int i, j, k;
@@ -506,7 +528,7 @@ __global__ void k_flags_ring(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int iv[3];
@@ -599,7 +621,7 @@ __global__ void k_init_uniform(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     const bool solid = isf[B.base * 2 + loc] == 0;
@@ -694,7 +716,7 @@ __global__ void k_init_fields(
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     const bool solid = isf[B.base * 2 + loc] == 0;
@@ -788,19 +810,21 @@ void build_ghost_map(const mrb_level *L, int depth, std::vector<GhostPair> &map)
     }
 }
 
-static int fill_boundary(mrb_level *L, void *arr, int ncomp, bool is_int, bool one_layer, hipStream_t s)
+static int fill_boundary(mrb_level *L, void *arr, int ncomp, bool is_int, bool one_layer, hipStream_t s,
+                         void *arr2 = nullptr)
 {
     const GhostPair *map = one_layer ? L->d_gmap1 : L->d_gmap;
     const int64_t n = one_layer ? L->n_gmap1 : L->n_gmap;
     if (n == 0) return MRB_OK;
+    const dim3 grid(nblocks(n), arr2 ? 2 : 1);
     if (is_int && ncomp == 2)
-        k_fill_map<int32_t, 2><<<nblocks(n), kBlock, 0, s>>>((int32_t *)arr, L->d_boxes, map, n);
+        k_fill_map<int32_t, 2><<<grid, kBlock, 0, s>>>((int32_t *)arr, (int32_t *)arr2, L->d_boxes, map, n);
     else if (!is_int && ncomp == NQ)
-        k_fill_map<double, NQ><<<nblocks(n), kBlock, 0, s>>>((double *)arr, L->d_boxes, map, n);
+        k_fill_map<double, NQ><<<grid, kBlock, 0, s>>>((double *)arr, (double *)arr2, L->d_boxes, map, n);
     else if (!is_int && ncomp == 3)
-        k_fill_map<double, 3><<<nblocks(n), kBlock, 0, s>>>((double *)arr, L->d_boxes, map, n);
+        k_fill_map<double, 3><<<grid, kBlock, 0, s>>>((double *)arr, (double *)arr2, L->d_boxes, map, n);
     else if (!is_int && ncomp == 19)
-        k_fill_map<double, 19><<<nblocks(n), kBlock, 0, s>>>((double *)arr, L->d_boxes, map, n);
+        k_fill_map<double, 19><<<grid, kBlock, 0, s>>>((double *)arr, (double *)arr2, L->d_boxes, map, n);
     else
         return set_error(MRB_E_ARG, "fill_boundary: unsupported component count");
     MRB_HIP(hipGetLastError());
@@ -812,10 +836,11 @@ int fab_fill_boundary(mrb_level *L, int lattice, hipStream_t s)
     return fill_boundary(L, L->pop[lattice][L->cur], NQ, false, false, s);
 }
 
-int fab_fill_boundary_map(mrb_level *L, int lattice, const GhostPair *map, int64_t n, hipStream_t s)
+int fab_fill_boundary_map(mrb_level *L, const GhostPair *map, int64_t n, hipStream_t s)
 {
     if (n == 0) return MRB_OK;
-    k_fill_map<double, NQ><<<nblocks(n), kBlock, 0, s>>>((double *)L->pop[lattice][L->cur], L->d_boxes, map, n);
+    k_fill_map<double, NQ><<<dim3(nblocks(n), 2), kBlock, 0, s>>>(
+        (double *)L->pop[0][L->cur], (double *)L->pop[1][L->cur], L->d_boxes, map, n);
     MRB_HIP(hipGetLastError());
     return MRB_OK;
 }
@@ -830,7 +855,7 @@ __global__ void k_fab_to_dense(const double *__restrict__ src, int ncomp, int co
 {
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    const int b = find_box(base, nbox, c);
+    const int b = find_box_flat(base, nbox, c);
     const BoxDev B = boxes[b];
     const int64_t loc = c - B.base;
     int i, j, k;
@@ -867,10 +892,8 @@ int fab_plot_fields(mrb_level *L, double *der, hipStream_t s)
 int fab_fill_boundary_depth(mrb_level *L, int depth, hipStream_t s)
 {
     const bool one = depth <= 1;
-    for (int l = 0; l < 2; ++l) {
-        const int rc = fill_boundary(L, L->pop[l][L->cur], NQ, false, one, s);
-        if (rc) return rc;
-    }
+    const int rc = fill_boundary(L, L->pop[0][L->cur], NQ, false, one, s, L->pop[1][L->cur]);
+    if (rc) return rc;
     L->fresh_depth = one ? 1 : L->ng;
     return MRB_OK;
 }
@@ -1897,7 +1920,7 @@ int mrb_stream(mrb_level *L, int lattice, void *stream)
     // through the spare buffer and copy back so that cur stays shared
     double *fin = (double *)L->pop[lattice][L->cur];
     double *fout = (double *)L->pop[lattice][1 - L->cur];
-    k_stream_fab<<<nblocks(L->total_cells), kBlock, 0, s>>>(fin, fout, L->d_isf, L->d_boxes, L->d_box_base,
+    k_stream_fab<<<nblocks(L->total_cells), kBlock, 0, s>>>(fin, fout, L->d_mask, L->d_boxes, L->d_box_base,
                                                             L->nbox, L->total_cells);
     MRB_HIP(hipGetLastError());
     std::swap(L->pop[lattice][0], L->pop[lattice][1]);
@@ -1927,9 +1950,7 @@ int mrb_collide(mrb_level *L, void *stream)
     k_eqrelax_fab<<<nb, kBlock, 0, s>>>(f, g, L->d_md, L->d_dq, L->d_isf, L->d_boxes, L->d_box_base,
                                         L->nbox, L->total_cells, L->cp);
     MRB_HIP(hipGetLastError());
-    rc = fill_boundary(L, f, NQ, false, false, s);
-    if (rc) return rc;
-    rc = fill_boundary(L, g, NQ, false, false, s);
+    rc = fill_boundary(L, f, NQ, false, false, s, g);
     if (rc) return rc;
     L->fresh_depth = L->ng;
     L->md_src = 1;
