@@ -346,6 +346,10 @@ struct mrb_level {
         int post_fresh_c = 0, post_fresh_f = 0;
     } amr_graph[2][2];
     hipStream_t cap_stream = nullptr;
+    mrb::GhostPair *d_gmap_in = nullptr;  // the 1-layer map grouped by offset beyond the box (k_fill_inward)
+    uint8_t *d_gmap_in_group = nullptr;   // per block of it: the offset
+    int64_t n_gmap_in = 0;
+    bool inward_fresh = false;  // between two steps of one mrb_advance: the pulled ghost components are filled
 };
 
 namespace mrb {
@@ -442,6 +446,8 @@ const char *compact_variant_name(int index);
 int fab_fill_boundary(mrb_level *L, int lattice, hipStream_t s);
 // FillBoundary of both lattices' current fab buffers over the given map
 int fab_fill_boundary_map(mrb_level *L, const GhostPair *map, int64_t n, hipStream_t s);
+// FillBoundary of both lattices, the first-layer components a batched step pulls
+int fab_fill_inward(mrb_level *L, hipStream_t s);
 // every ghost cell (within `depth` layers) that FillBoundary writes, with its owner
 void build_ghost_map(const mrb_level *L, int depth, std::vector<GhostPair> &map);
 // FillBoundary of both lattices, `depth` ghost layers (1 or ng); sets fresh_depth

@@ -117,6 +117,48 @@ __global__ void k_fill_map(
     static_for<NC>([&](auto cc) { dst[decltype(cc)::value * dn] = v[decltype(cc)::value]; });
 }
 
+// FillBoundary of what a batched step's pulls read: a first-layer ghost beyond
+// the box by o (o_d in -1, 0, 1) only feeds valid cells through the directions
+// that point inward, c_d = -o_d where o_d is not 0 -- 9 of the 27 beyond a
+// face, 3 beyond an edge, 1 beyond a corner.  Entries are grouped by o, each
+// group padded to whole blocks (entries with dst_box < 0), so that a block's
+// component list is known at compile time.  Both lattices (blockIdx.y).
+// 128x96x72 in 32^3 boxes: 134 us for all components of both lattices.
+template <int OX, int OY, int OZ>
+__device__ __forceinline__ void fill_inward(double *__restrict__ arr, const BoxDev &D, const BoxDev &S,
+                                            const GhostPair &p)
+{
+    double *dst = arr + D.base * NQ + p.dst_local;
+    const double *src = arr + S.base * NQ + p.src_local;
+    double v[NQ];
+    static_for<NQ>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr ((OX == 0 || ev(q, 0) == -OX) && (OY == 0 || ev(q, 1) == -OY) && (OZ == 0 || ev(q, 2) == -OZ))
+            v[q] = src[int64_t(q) * S.ncell];
+    });
+    static_for<NQ>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr ((OX == 0 || ev(q, 0) == -OX) && (OY == 0 || ev(q, 1) == -OY) && (OZ == 0 || ev(q, 2) == -OZ))
+            dst[int64_t(q) * D.ncell] = v[q];
+    });
+}
+__global__ void __launch_bounds__(kBlock) k_fill_inward(
+    double *__restrict__ f, double *__restrict__ g, const BoxDev *__restrict__ boxes,
+    const GhostPair *__restrict__ map, const uint8_t *__restrict__ group)
+{
+    const uint32_t block = xcd_index(blockIdx.x, gridDim.x);
+    const GhostPair p = map[int64_t(block) * kBlock + threadIdx.x];
+    if (p.dst_box < 0) return;
+    double *arr = blockIdx.y ? g : f;
+    const int o = group[block];  // (o_z + 1) * 9 + (o_y + 1) * 3 + o_x + 1
+    static_for<27>([&](auto oc) {
+        constexpr int k = decltype(oc)::value;
+        if constexpr (k != 13) {
+            if (o == k) fill_inward<k % 3 - 1, k / 3 % 3 - 1, k / 9 - 1>(arr, boxes[p.dst_box], boxes[p.src_box], p);
+        }
+    });
+}
+
 // ---------------------------------------------------------------------------
 // LBM::stream (LBM.cpp:558-604) as a pull over every fab cell y:
 //   y fluid and y-c_p inside the fab:  fluid(y-c_p) ? f_p(y-c_p) : f_pbar(y)
@@ -313,48 +355,8 @@ __global__ void k_moments_fab(
     o[18 * s] = M.T;
 }
 
-// ---------------------------------------------------------------------------
-// LBM::compute_q_corrections (LBM.cpp:959-991), valid cells
-// ---------------------------------------------------------------------------
-__global__ void k_dq_fab(
-    const double *__restrict__ md, const int32_t *__restrict__ isf, double *__restrict__ dq,
-    const BoxDev *__restrict__ boxes, const int64_t *__restrict__ base, int nbox, int64_t total,
-    int n0, int n1, int n2, CollideParams P)
-{
-    const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= total) return;
-    const int b = find_box_flat(base, nbox, c);
-    const BoxDev B = boxes[b];
-    const int64_t loc = c - B.base;
-    int iv[3];
-    local_to_ijk(B, loc, iv[0], iv[1], iv[2]);
-    if (!in_valid(B, iv[0], iv[1], iv[2])) return;
-    const int32_t *fl = isf + B.base * 2;
-    if (fl[loc] != 1) return;
-    const double *m = md + B.base * 19;
-    const int nd[3] = {n0, n1, n2};
-    for (int d = 0; d < 3; ++d) {
-        int p[3] = {iv[0], iv[1], iv[2]}, q[3] = {iv[0], iv[1], iv[2]};
-        p[d] += 1;
-        q[d] -= 1;
-        const bool p_ok = p[d] >= 0 && p[d] < nd[d] && p[(d + 1) % 3] >= 0 &&
-                          p[(d + 1) % 3] < nd[(d + 1) % 3] && p[(d + 2) % 3] >= 0 &&
-                          p[(d + 2) % 3] < nd[(d + 2) % 3] &&
-                          fl[loc_of(B, p[0], p[1], p[2])] == 1;
-        const bool m_ok = q[d] >= 0 && q[d] < nd[d] && q[(d + 1) % 3] >= 0 &&
-                          q[(d + 1) % 3] < nd[(d + 1) % 3] && q[(d + 2) % 3] >= 0 &&
-                          q[(d + 2) % 3] < nd[(d + 2) % 3] &&
-                          fl[loc_of(B, q[0], q[1], q[2])] == 1;
-        const int comp = 6 + d;
-        const double qp = p_ok ? m[comp * B.ncell + loc_of(B, p[0], p[1], p[2])] : 0.0;
-        const double qm = m_ok ? m[comp * B.ncell + loc_of(B, q[0], q[1], q[2])] : 0.0;
-        const double qcv = m[comp * B.ncell + loc];
-        dq[B.base * 3 + d * B.ncell + loc] = one_sided_gradient(p_ok, m_ok, qp, qcv, qm, P.inv_dx[d]);
-    }
-}
-
 // gradient() (Utilities.H:279-312) of macrodata component comp along d at
-// the valid fluid cell iv of box B, as k_dq_fab takes it: a neighbour counts
+// the valid fluid cell iv of box B: a neighbour counts
 // where it lies inside the domain box and is fluid
 __device__ double fab_gradient(const double *__restrict__ m, const int32_t *__restrict__ fl, const BoxDev &B,
                                const int iv[3], int d, int comp, const int nd[3], double inv_dx)
@@ -413,44 +415,31 @@ __global__ void k_plot_derived_fab(
 }
 
 // ---------------------------------------------------------------------------
-// macrodata_to_equilibrium + relax_f_to_equilibrium (LBM.cpp:621-807),
-// valid fluid cells, in place
+// compute_q_corrections (LBM.cpp:959-991), macrodata_to_equilibrium and
+// relax_f_to_equilibrium (LBM.cpp:621-807), valid fluid cells, in place.
+// Blocks take the batched step's tiles, so that no lane idles on a ghost (two
+// in five fab cells of a 32^3 box with three layers are valid); the moments
+// come from the cell's own populations, which are read anyway, as
+// k_moments_fab formed them, and only the neighbours' QCorr from md.  The
+// gradient in a pass of its own and the moments read back: 177 us at 90x72x56
+// in 32^3 boxes.
 // ---------------------------------------------------------------------------
-__global__ void k_eqrelax_fab(
-    double *__restrict__ f, double *__restrict__ g, const double *__restrict__ md,
-    const double *__restrict__ dq, const int32_t *__restrict__ isf,
-    const BoxDev *__restrict__ boxes, const int64_t *__restrict__ base, int nbox, int64_t total,
-    CollideParams P)
+__global__ void __launch_bounds__(kFabTile) k_eqrelax_fab(
+    double *__restrict__ f, double *__restrict__ g, const double *__restrict__ md, const int32_t *__restrict__ isf,
+    const BoxDev *__restrict__ boxes, const FabTile *__restrict__ tiles, int n0, int n1, int n2, CollideParams P)
 {
-    const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= total) return;
-    const int b = find_box_flat(base, nbox, c);
-    const BoxDev B = boxes[b];
-    const int64_t loc = c - B.base;
-    int i, j, k;
-    local_to_ijk(B, loc, i, j, k);
-    if (!in_valid(B, i, j, k)) return;
-    if (isf[B.base * 2 + loc] != 1) return;
+    const FabTile tile = tiles[blockIdx.x];
+    const BoxDev &B = boxes[tile.box];
+    const uint32_t rx = uint32_t(B.vhi[0] - B.vlo[0] + 1), ry = uint32_t(B.vhi[1] - B.vlo[1] + 1),
+                   rz = uint32_t(B.vhi[2] - B.vlo[2] + 1);
+    const uint32_t c = uint32_t(tile.first) + threadIdx.x;
+    if (c >= rx * ry * rz) return;
+    const uint32_t kk = c / (rx * ry), rem = c - kk * rx * ry, jj = rem / rx;
+    const int iv[3] = {B.vlo[0] + int(rem - jj * rx), B.vlo[1] + int(jj), B.vlo[2] + int(kk)};
+    const int64_t loc = loc_of(B, iv[0], iv[1], iv[2]);
+    const int32_t *fl = isf + B.base * 2;
+    if (fl[loc] != 1) return;
     const int64_t s = B.ncell;
-    const double *m = md + B.base * 19 + loc;
-    Moments mo;
-    mo.rho = m[0];
-    mo.E = m[5 * s];
-    mo.pxx = m[9 * s];
-    mo.pyy = m[10 * s];
-    mo.pzz = m[11 * s];
-    mo.pxy = m[12 * s];
-    mo.pxz = m[13 * s];
-    mo.pyz = m[14 * s];
-    mo.qx = m[15 * s];
-    mo.qy = m[16 * s];
-    mo.qz = m[17 * s];
-    Macro M;
-    M.u = m[1 * s];
-    M.v = m[2 * s];
-    M.w = m[3 * s];
-    M.T = m[18 * s];
-    const double *d = dq + B.base * 3 + loc;
     double *fp = f + B.base * NQ + loc;
     double *gp = g + B.base * NQ + loc;
     double fv[NQ], gv[NQ];
@@ -458,7 +447,15 @@ __global__ void k_eqrelax_fab(
         fv[q] = fp[q * s];
         gv[q] = gp[q * s];
     }
-    collide_cell(fv, gv, mo, M, d[0], d[s], d[2 * s], P, [&](auto qc, double fo, double go) {
+    const double *m = md + B.base * 19;
+    const int nd[3] = {n0, n1, n2};
+    const double dqx = fab_gradient(m, fl, B, iv, 0, 6, nd, P.inv_dx[0]);
+    const double dqy = fab_gradient(m, fl, B, iv, 1, 7, nd, P.inv_dx[1]);
+    const double dqz = fab_gradient(m, fl, B, iv, 2, 8, nd, P.inv_dx[2]);
+    Moments mo;
+    accumulate_moments(fv, gv, mo);
+    const Macro M = macro_from(mo.rho, mo.jx, mo.jy, mo.jz, mo.E, P);
+    collide_cell(fv, gv, mo, M, dqx, dqy, dqz, P, [&](auto qc, double fo, double go) {
         constexpr int q = decltype(qc)::value;
         fp[q * s] = fo;
         gp[q * s] = go;
@@ -845,6 +842,15 @@ int fab_fill_boundary_map(mrb_level *L, const GhostPair *map, int64_t n, hipStre
     return MRB_OK;
 }
 
+int fab_fill_inward(mrb_level *L, hipStream_t s)
+{
+    if (L->n_gmap_in == 0) return MRB_OK;
+    k_fill_inward<<<dim3(unsigned(L->n_gmap_in / kBlock), 2), kBlock, 0, s>>>(
+        (double *)L->pop[0][L->cur], (double *)L->pop[1][L->cur], L->d_boxes, L->d_gmap_in, L->d_gmap_in_group);
+    MRB_HIP(hipGetLastError());
+    return MRB_OK;
+}
+
 int fab_fill_boundary_q(mrb_level *L, hipStream_t s) { return fill_boundary(L, L->d_dq, 3, false, true, s); }
 
 // one fab component over the valid cells into a domain-sized array
@@ -1188,6 +1194,34 @@ int mrb_level_create(const mrb_level_desc *desc, mrb_level **out)
             MRB_HIP(hipMalloc(&L->d_gmap1, sizeof(GhostPair) * map.size()));
             MRB_HIP(hipMemcpy(L->d_gmap1, map.data(), sizeof(GhostPair) * map.size(), hipMemcpyHostToDevice));
         }
+        // the same, grouped by the offset beyond the box (k_fill_inward)
+        std::vector<GhostPair> by_offset[27];
+        for (const GhostPair &p : map) {
+            const BoxDev &B = L->boxes[size_t(p.dst_box)];
+            const int64_t nxy = int64_t(B.n[0]) * B.n[1];
+            const int c[3] = {int(p.dst_local % B.n[0]), int((p.dst_local % nxy) / B.n[0]), int(p.dst_local / nxy)};
+            int o = 0;
+            for (int d = 2; d >= 0; --d) {
+                const int g = B.lo[d] + c[d];
+                o = o * 3 + (g < B.vlo[d] ? 0 : (g > B.vhi[d] ? 2 : 1));
+            }
+            by_offset[o].push_back(p);
+        }
+        std::vector<GhostPair> grouped;
+        std::vector<uint8_t> group;
+        for (int o = 0; o < 27; ++o) {
+            grouped.insert(grouped.end(), by_offset[o].begin(), by_offset[o].end());
+            while (grouped.size() % kBlock) grouped.push_back(GhostPair{-1, -1, 0, 0});
+            group.resize(grouped.size() / kBlock, uint8_t(o));
+        }
+        L->n_gmap_in = int64_t(grouped.size());
+        if (!grouped.empty()) {
+            MRB_HIP(hipMalloc(&L->d_gmap_in, sizeof(GhostPair) * grouped.size()));
+            MRB_HIP(hipMemcpy(L->d_gmap_in, grouped.data(), sizeof(GhostPair) * grouped.size(),
+                              hipMemcpyHostToDevice));
+            MRB_HIP(hipMalloc(&L->d_gmap_in_group, group.size()));
+            MRB_HIP(hipMemcpy(L->d_gmap_in_group, group.data(), group.size(), hipMemcpyHostToDevice));
+        }
         MRB_HIP(hipMalloc(&L->d_mask, sizeof(uint32_t) * T));
         MRB_HIP(hipMemset(L->d_mask, 0, sizeof(uint32_t) * T));
         std::vector<FabTile> tiles;
@@ -1306,6 +1340,8 @@ int mrb_level_destroy(mrb_level *L)
         if (e) (void)hipEventDestroy(e);
     (void)hipFree(L->d_gmap);
     (void)hipFree(L->d_gmap1);
+    (void)hipFree(L->d_gmap_in);
+    (void)hipFree(L->d_gmap_in_group);
     (void)hipFree(L->d_bcells);
     (void)hipFree(L->d_sweep_q);
     (void)hipFree(L->d_sweep_qx);
@@ -1944,11 +1980,8 @@ int mrb_collide(mrb_level *L, void *stream)
     MRB_HIP(hipGetLastError());
     int rc = fill_boundary(L, L->d_md, 19, false, true, s);
     if (rc) return rc;
-    k_dq_fab<<<nb, kBlock, 0, s>>>(L->d_md, L->d_isf, L->d_dq, L->d_boxes, L->d_box_base, L->nbox,
-                                   L->total_cells, L->ncell[0], L->ncell[1], L->ncell[2], L->cp);
-    MRB_HIP(hipGetLastError());
-    k_eqrelax_fab<<<nb, kBlock, 0, s>>>(f, g, L->d_md, L->d_dq, L->d_isf, L->d_boxes, L->d_box_base,
-                                        L->nbox, L->total_cells, L->cp);
+    k_eqrelax_fab<<<unsigned(L->n_tiles_c), kFabTile, 0, s>>>(f, g, L->d_md, L->d_isf, L->d_boxes, L->d_tiles_c,
+                                                              L->ncell[0], L->ncell[1], L->ncell[2], L->cp);
     MRB_HIP(hipGetLastError());
     rc = fill_boundary(L, f, NQ, false, false, s, g);
     if (rc) return rc;
@@ -1958,6 +1991,24 @@ int mrb_collide(mrb_level *L, void *stream)
 }
 
 // ---- hot path --------------------------------------------------------------
+
+// a batched step of a single fab level; last: its first ghost layer is filled
+// in every component, else in those the next step pulls
+static int fab_single_step(mrb_level *L, bool last, hipStream_t s)
+{
+    int rc;
+    // the batched step pulls ring 1 only: FillBoundary one layer deep
+    if (L->fresh_depth < 1 && !L->inward_fresh && (rc = fab_fill_boundary_depth(L, 1, s))) return rc;
+    L->inward_fresh = false;
+    for (int l = 0; l < 2; ++l)
+        if ((rc = mrb_physbc(L, l, s))) return rc;
+    if ((rc = fab_batched_step(L, nullptr, last ? 1 : 0, s))) return rc;
+    if (!last) {
+        if ((rc = fab_fill_inward(L, s))) return rc;
+        L->inward_fresh = true;  // (until the next step of the same call)
+    }
+    return MRB_OK;
+}
 
 int mrb_stream_collide(mrb_level *L, void *stream)
 {
@@ -1976,17 +2027,19 @@ int mrb_stream_collide(mrb_level *L, void *stream)
             if ((rc = mrb_stream(L, l, stream))) return rc;
         return mrb_collide(L, stream);
     }
-    // the batched step pulls ring 1 only: FillBoundary one layer deep
-    if (L->fresh_depth < 1 && (rc = fab_fill_boundary_depth(L, 1, as_stream(stream)))) return rc;
-    for (int l = 0; l < 2; ++l)
-        if ((rc = mrb_physbc(L, l, stream))) return rc;
-    return fab_batched_step(L, nullptr, 1, as_stream(stream));
+    return fab_single_step(L, true, as_stream(stream));
 }
 
 int mrb_advance(mrb_level *L, int nsteps, void *stream)
 {
+    // between the steps of one call on a fully periodic fab level only the
+    // components that the next step pulls are filled (the boundary functor of
+    // a non-periodic face reads others); the last step leaves the first ghost
+    // layer as mrb_stream_collide does
+    const bool inward = L && L->layout == MRB_LAYOUT_FAB && L->flags_ready && L->ng >= 2 && !L->amr_crse &&
+                        L->n_bcells == 0;
     for (int n = 0; n < nsteps; ++n) {
-        const int rc = mrb_stream_collide(L, stream);
+        const int rc = inward ? fab_single_step(L, n == nsteps - 1, as_stream(stream)) : mrb_stream_collide(L, stream);
         if (rc) return rc;
     }
     return MRB_OK;
