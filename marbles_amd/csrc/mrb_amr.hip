@@ -147,11 +147,18 @@ __global__ void __launch_bounds__(kAmrBlock) k_explode_slopes(
 __global__ void __launch_bounds__(kAmrBlock) k_explode_groups(
     const double *__restrict__ crse_f, const double *__restrict__ crse_g, double *__restrict__ fine_f,
     double *__restrict__ fine_g, const BoxDev *__restrict__ cboxes, const BoxDev *__restrict__ fboxes,
-    const ExplodeGroup *__restrict__ groups, int64_t n)
+    const ExplodeGroup *__restrict__ groups, int64_t n, int pulled_only)
 {
     const int64_t t = int64_t(xcd_index(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const int q = int(blockIdx.y);
+    if (pulled_only) {
+        // ring-3 children only feed the ghost stream of rings 1 and 2 through
+        // the directions that point inward
+        const int r3 = groups[t].ring3;
+        for (int d = 0; d < 3; ++d)
+            if (((r3 >> (2 * d)) & 1 && kEV[q][d] != 1) || ((r3 >> (2 * d + 1)) & 1 && kEV[q][d] != -1)) return;
+    }
     const double *crse = blockIdx.z ? crse_g : crse_f;
     double *fine = blockIdx.z ? fine_g : fine_f;
     const ExplodeGroup G = groups[t];
@@ -375,7 +382,11 @@ void amr_release(mrb_level *L)
     L->d_qring = nullptr;
     if (L->d_gmap_step) (void)hipFree(L->d_gmap_step);
     L->d_gmap_step = nullptr;
-    L->n_gmap_step = 0;
+    L->n_gmap_step = L->n_gmap_step_full = L->n_gmap_step_in = 0;
+    if (L->d_gmap_step_in) (void)hipFree(L->d_gmap_step_in);
+    if (L->d_gmap_step_in_group) (void)hipFree(L->d_gmap_step_in_group);
+    L->d_gmap_step_in = nullptr;
+    L->d_gmap_step_in_group = nullptr;
     L->n_expl_le2 = 0;
     if (L->d_coal_has) (void)hipFree(L->d_coal_has);
     L->d_coal = L->d_expl = nullptr;
@@ -536,6 +547,16 @@ int mrb_amr_link(mrb_level *crse, mrb_level *fine)
                 G.crse_local = e.crse_local;
                 G.crse_box = e.crse_box;
                 G.flags = parents.list[size_t(e.parent)].flags;
+                // a group's children in the third layer beyond a side of the
+                // (coarse-aligned) box all lie in it
+                const BoxDev &FB = fine->boxes[e.fine_box];
+                const int64_t nxy = int64_t(FB.n[0]) * FB.n[1];
+                const int c[3] = {int(e.fine_local % FB.n[0]), int((e.fine_local % nxy) / FB.n[0]),
+                                  int(e.fine_local / nxy)};
+                for (int d = 0; d < 3; ++d) {
+                    if (FB.lo[d] + c[d] >= FB.vhi[d] + 3) G.ring3 |= 2 << (2 * d);
+                    if (FB.lo[d] + c[d] <= FB.vlo[d] - 3) G.ring3 |= 1 << (2 * d);
+                }
                 groups.push_back(G);
             }
             groups.back().children |= 1 << (e.bits & 7);
@@ -564,7 +585,7 @@ int mrb_amr_link(mrb_level *crse, mrb_level *fine)
     // listed ghost stream and Q pass pull its 26 neighbours) or within the
     // ghost depth of a non-periodic domain face (the boundary functor).
     // The other deeper ghosts keep the values of the last full fill.
-    std::vector<GhostPair> step_map;
+    std::vector<GhostPair> step_map, step_in;
     {
         std::vector<uint8_t> need(size_t(fine->total_cells), 0);
         auto fab_ijk = [](const BoxDev &B, int64_t loc, int c[3]) {
@@ -598,9 +619,19 @@ int mrb_amr_link(mrb_level *crse, mrb_level *fine)
                 layer = std::max(layer, std::max(FB.vlo[d] - g, g - FB.vhi[d]));
                 if (!fine->periodic[d] && (g < fine->ng || g >= fine->ncell[d] - fine->ng)) near_face = true;
             }
-            if (layer <= 1 || near_face || need[size_t(FB.base + p.dst_local)]) step_map.push_back(p);
+            if (near_face || need[size_t(FB.base + p.dst_local)])
+                step_map.push_back(p);
+            else if (layer <= 1)
+                step_in.push_back(p);
         }
     }
+    // (the entries whose ghosts only valid cells pull come last, and again
+    // grouped for the fill of their pulled components)
+    const int64_t n_step_full = int64_t(step_map.size());
+    step_map.insert(step_map.end(), step_in.begin(), step_in.end());
+    std::vector<GhostPair> step_grouped;
+    std::vector<uint8_t> step_group;
+    group_by_offset(fine, step_in, step_grouped, step_group);
     // per coarse fab cell: the coalescence entry of valid cells under the
     // fine footprint or its ring
     std::vector<int32_t> coal_cell(size_t(crse->total_cells), -1);
@@ -651,6 +682,15 @@ int mrb_amr_link(mrb_level *crse, mrb_level *fine)
                           hipMemcpyHostToDevice));
     }
     fine->n_gmap_step = int64_t(step_map.size());
+    fine->n_gmap_step_full = n_step_full;
+    fine->n_gmap_step_in = int64_t(step_grouped.size());
+    if (!step_grouped.empty()) {
+        MRB_HIP(hipMalloc(&fine->d_gmap_step_in, sizeof(GhostPair) * step_grouped.size()));
+        MRB_HIP(hipMemcpy(fine->d_gmap_step_in, step_grouped.data(), sizeof(GhostPair) * step_grouped.size(),
+                          hipMemcpyHostToDevice));
+        MRB_HIP(hipMalloc(&fine->d_gmap_step_in_group, step_group.size()));
+        MRB_HIP(hipMemcpy(fine->d_gmap_step_in_group, step_group.data(), step_group.size(), hipMemcpyHostToDevice));
+    }
     if (!qring.empty()) {
         MRB_HIP(hipMalloc(&fine->d_qring, sizeof(ExplodeEntry) * qring.size()));
         MRB_HIP(hipMemcpy(fine->d_qring, qring.data(), sizeof(ExplodeEntry) * qring.size(), hipMemcpyHostToDevice));
@@ -689,15 +729,17 @@ int mrb_coalesce(const mrb_level *fine, mrb_level *crse, void *stream)
 
 namespace mrb {
 // fine ghosts over uncovered domain from the coarse level, lattices
-// first .. first + count - 1, then the boundary functor
-static int explode_uncovered(const mrb_level *crse, mrb_level *fine, int first, int count, hipStream_t s)
+// first .. first + count - 1, then the boundary functor; pulled_only: of the
+// third layer only the components that the two-level step reads
+static int explode_uncovered(const mrb_level *crse, mrb_level *fine, int first, int count, bool pulled_only,
+                             hipStream_t s)
 {
     if (fine->n_expl_groups > 0) {
         const int last = first + count - 1;
         k_explode_groups<<<dim3(blocks_for(fine->n_expl_groups), NQ, unsigned(count)), kAmrBlock, 0, s>>>(
             (const double *)crse->pop[first][crse->cur], (const double *)crse->pop[last][crse->cur],
             (double *)fine->pop[first][fine->cur], (double *)fine->pop[last][fine->cur], crse->d_boxes, fine->d_boxes,
-            (const ExplodeGroup *)fine->d_expl_groups, fine->n_expl_groups);
+            (const ExplodeGroup *)fine->d_expl_groups, fine->n_expl_groups, pulled_only ? 1 : 0);
         MRB_HIP(hipGetLastError());
     }
     for (int l = first; l < first + count; ++l) {
@@ -716,11 +758,19 @@ static int explode_coarse_ghosts(const mrb_level *crse, const mrb_level *fine, h
 }
 // the fine FillBoundary of the two-level step, both lattices: what the step
 // reads (the linked pair's step map) rather than every ghost layer
-static int fill_fine_step(mrb_level *fine, hipStream_t s)
+// (pulled_only: of a first-layer ghost that no ghost stream reads only the
+// components that valid cells pull)
+static int fill_fine_step(mrb_level *fine, bool pulled_only, hipStream_t s)
 {
     const bool part = fine->d_gmap_step != nullptr;
-    const int rc = part ? fab_fill_boundary_map(fine, fine->d_gmap_step, fine->n_gmap_step, s)
-                        : fab_fill_boundary_depth(fine, fine->ng, s);
+    int rc;
+    if (part && pulled_only) {
+        rc = fab_fill_boundary_map(fine, fine->d_gmap_step, fine->n_gmap_step_full, s);
+        if (!rc) rc = fab_fill_inward(fine, fine->d_gmap_step_in, fine->d_gmap_step_in_group, fine->n_gmap_step_in, s);
+    } else {
+        rc = part ? fab_fill_boundary_map(fine, fine->d_gmap_step, fine->n_gmap_step, s)
+                  : fab_fill_boundary_depth(fine, fine->ng, s);
+    }
     if (rc) return rc;
     fine->fresh_depth = part ? 1 : fine->ng;
     return MRB_OK;
@@ -740,7 +790,7 @@ int mrb_explode(const mrb_level *crse, mrb_level *fine, int lattice, void *strea
     if (!rc) rc = fab_fill_boundary(fine, lattice, s);
     if (rc) return rc;
     if (lattice == 1) fine->fresh_depth = fine->ng;
-    return explode_uncovered(crse, fine, lattice, 1, s);
+    return explode_uncovered(crse, fine, lattice, 1, false, s);
 }
 
 static int check_advance(mrb_level *crse, mrb_level *fine)
@@ -759,18 +809,22 @@ static int check_advance(mrb_level *crse, mrb_level *fine)
 // uncovered ghosts are streamed from up to ng layers during the first
 // substep; after the second substep nothing reads fine ghosts covered by
 // fine boxes (the coalescence takes those cells' children from the owning
-// box) before the next explosion refills them.
-static int amr_step(mrb_level *crse, mrb_level *fine, void *stream)
+// box) before the next explosion refills them.  last: the call's last step,
+// which fills the ghost components that it reads no more than the others did
+// but that a caller may look at; the steps before it leave them out (not with
+// non-periodic faces, whose boundary functor reads them).
+static int amr_step(mrb_level *crse, mrb_level *fine, bool last, void *stream)
 {
     int rc;
     hipStream_t s = as_stream(stream);
+    const bool pulled_only = !last && fine->n_bcells == 0 && fine->ng == 3;
     const int depth = std::max(1, fine->expl_crse_depth);
     if (crse->fresh_depth < depth && (rc = fab_fill_boundary_depth(crse, depth, s))) return rc;
     for (int l = 0; l < 2; ++l)
         if ((rc = mrb_physbc(crse, l, stream))) return rc;
     if ((rc = explode_coarse_ghosts(crse, fine, s))) return rc;
-    if ((rc = fill_fine_step(fine, s))) return rc;
-    if ((rc = explode_uncovered(crse, fine, 0, 2, s))) return rc;
+    if ((rc = fill_fine_step(fine, pulled_only, s))) return rc;
+    if ((rc = explode_uncovered(crse, fine, 0, 2, pulled_only, s))) return rc;
     for (int sub = 0; sub < 2; ++sub) {
         for (int l = 0; l < 2; ++l)
             if ((rc = mrb_physbc(fine, l, stream))) return rc;
@@ -781,7 +835,7 @@ static int amr_step(mrb_level *crse, mrb_level *fine, void *stream)
         fine->stream_substep = 0;
         if (rc) return rc;
         // the ghosts the second substep reads
-        if (sub == 0 && (rc = fill_fine_step(fine, s))) return rc;
+        if (sub == 0 && (rc = fill_fine_step(fine, pulled_only, s))) return rc;
     }
     // advance(0): stream, average_down_to, collide, with the coalescence
     // fused into the coarse passes
@@ -1028,7 +1082,7 @@ int mrb_amr_advance(mrb_level *crse, mrb_level *fine, int nsteps, void *stream)
     int rc = check_advance(crse, fine);
     if (rc) return rc;
     for (int n = 0; n < nsteps; ++n)
-        if ((rc = amr_step(crse, fine, stream))) return rc;
+        if ((rc = amr_step(crse, fine, n == nsteps - 1, stream))) return rc;
     return MRB_OK;
 }
 
@@ -1052,7 +1106,7 @@ int mrb_amr_advance_graph(mrb_level *crse, mrb_level *fine, int nsteps, void *st
             G.gen_f = fine->gen;
             G.fine_cur = cur_f;
             MRB_HIP(hipStreamBeginCapture(fine->cap_stream, hipStreamCaptureModeThreadLocal));
-            rc = amr_step(crse, fine, fine->cap_stream);
+            rc = amr_step(crse, fine, true, fine->cap_stream);
             hipGraph_t graph = nullptr;
             const hipError_t ec = hipStreamEndCapture(fine->cap_stream, &graph);
             G.post_cur_c = crse->cur;

@@ -137,6 +137,7 @@ struct ExplodeGroup {
     int64_t crse_local, fine_local;
     int32_t crse_box, fine_box;
     int32_t flags, children;
+    int32_t ring3;  // bit 2d / 2d+1: the children lie in the third layer beyond the low / high side
 };
 
 // Single-pass z-sweep kernel shapes: rows per tile and z planes per chunk.
@@ -349,6 +350,11 @@ struct mrb_level {
     mrb::GhostPair *d_gmap_in = nullptr;  // the 1-layer map grouped by offset beyond the box (k_fill_inward)
     uint8_t *d_gmap_in_group = nullptr;   // per block of it: the offset
     int64_t n_gmap_in = 0;
+    // fine level of a linked pair: d_gmap_step's first n_gmap_step_full entries
+    // are read in every component; the rest again, grouped for k_fill_inward
+    int64_t n_gmap_step_full = 0, n_gmap_step_in = 0;
+    mrb::GhostPair *d_gmap_step_in = nullptr;
+    uint8_t *d_gmap_step_in_group = nullptr;
     bool inward_fresh = false;  // between two steps of one mrb_advance: the pulled ghost components are filled
 };
 
@@ -446,8 +452,13 @@ const char *compact_variant_name(int index);
 int fab_fill_boundary(mrb_level *L, int lattice, hipStream_t s);
 // FillBoundary of both lattices' current fab buffers over the given map
 int fab_fill_boundary_map(mrb_level *L, const GhostPair *map, int64_t n, hipStream_t s);
-// FillBoundary of both lattices, the first-layer components a batched step pulls
-int fab_fill_inward(mrb_level *L, hipStream_t s);
+// FillBoundary of both lattices over a grouped first-layer map (n entries, a
+// multiple of the block), the components a batched step pulls
+int fab_fill_inward(mrb_level *L, const GhostPair *map, const uint8_t *group, int64_t n, hipStream_t s);
+// first-layer entries grouped by their offset beyond the box, each group padded
+// to whole blocks; per block its offset
+void group_by_offset(const mrb_level *L, const std::vector<GhostPair> &map, std::vector<GhostPair> &grouped,
+                     std::vector<uint8_t> &group);
 // every ghost cell (within `depth` layers) that FillBoundary writes, with its owner
 void build_ghost_map(const mrb_level *L, int depth, std::vector<GhostPair> &map);
 // FillBoundary of both lattices, `depth` ghost layers (1 or ng); sets fresh_depth

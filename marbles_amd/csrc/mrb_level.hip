@@ -807,6 +807,28 @@ void build_ghost_map(const mrb_level *L, int depth, std::vector<GhostPair> &map)
     }
 }
 
+void group_by_offset(const mrb_level *L, const std::vector<GhostPair> &map, std::vector<GhostPair> &grouped,
+                     std::vector<uint8_t> &group)
+{
+    std::vector<GhostPair> by_offset[27];
+    for (const GhostPair &p : map) {
+        const BoxDev &B = L->boxes[size_t(p.dst_box)];
+        const int64_t nxy = int64_t(B.n[0]) * B.n[1];
+        const int c[3] = {int(p.dst_local % B.n[0]), int((p.dst_local % nxy) / B.n[0]), int(p.dst_local / nxy)};
+        int o = 0;
+        for (int d = 2; d >= 0; --d) {
+            const int g = B.lo[d] + c[d];
+            o = o * 3 + (g < B.vlo[d] ? 0 : (g > B.vhi[d] ? 2 : 1));
+        }
+        by_offset[o].push_back(p);
+    }
+    for (int o = 0; o < 27; ++o) {
+        grouped.insert(grouped.end(), by_offset[o].begin(), by_offset[o].end());
+        while (grouped.size() % kBlock) grouped.push_back(GhostPair{-1, -1, 0, 0});
+        group.resize(grouped.size() / kBlock, uint8_t(o));
+    }
+}
+
 static int fill_boundary(mrb_level *L, void *arr, int ncomp, bool is_int, bool one_layer, hipStream_t s,
                          void *arr2 = nullptr)
 {
@@ -842,11 +864,11 @@ int fab_fill_boundary_map(mrb_level *L, const GhostPair *map, int64_t n, hipStre
     return MRB_OK;
 }
 
-int fab_fill_inward(mrb_level *L, hipStream_t s)
+int fab_fill_inward(mrb_level *L, const GhostPair *map, const uint8_t *group, int64_t n, hipStream_t s)
 {
-    if (L->n_gmap_in == 0) return MRB_OK;
-    k_fill_inward<<<dim3(unsigned(L->n_gmap_in / kBlock), 2), kBlock, 0, s>>>(
-        (double *)L->pop[0][L->cur], (double *)L->pop[1][L->cur], L->d_boxes, L->d_gmap_in, L->d_gmap_in_group);
+    if (n == 0) return MRB_OK;
+    k_fill_inward<<<dim3(unsigned(n / kBlock), 2), kBlock, 0, s>>>((double *)L->pop[0][L->cur],
+                                                                  (double *)L->pop[1][L->cur], L->d_boxes, map, group);
     MRB_HIP(hipGetLastError());
     return MRB_OK;
 }
@@ -1195,25 +1217,9 @@ int mrb_level_create(const mrb_level_desc *desc, mrb_level **out)
             MRB_HIP(hipMemcpy(L->d_gmap1, map.data(), sizeof(GhostPair) * map.size(), hipMemcpyHostToDevice));
         }
         // the same, grouped by the offset beyond the box (k_fill_inward)
-        std::vector<GhostPair> by_offset[27];
-        for (const GhostPair &p : map) {
-            const BoxDev &B = L->boxes[size_t(p.dst_box)];
-            const int64_t nxy = int64_t(B.n[0]) * B.n[1];
-            const int c[3] = {int(p.dst_local % B.n[0]), int((p.dst_local % nxy) / B.n[0]), int(p.dst_local / nxy)};
-            int o = 0;
-            for (int d = 2; d >= 0; --d) {
-                const int g = B.lo[d] + c[d];
-                o = o * 3 + (g < B.vlo[d] ? 0 : (g > B.vhi[d] ? 2 : 1));
-            }
-            by_offset[o].push_back(p);
-        }
         std::vector<GhostPair> grouped;
         std::vector<uint8_t> group;
-        for (int o = 0; o < 27; ++o) {
-            grouped.insert(grouped.end(), by_offset[o].begin(), by_offset[o].end());
-            while (grouped.size() % kBlock) grouped.push_back(GhostPair{-1, -1, 0, 0});
-            group.resize(grouped.size() / kBlock, uint8_t(o));
-        }
+        group_by_offset(L.get(), map, grouped, group);
         L->n_gmap_in = int64_t(grouped.size());
         if (!grouped.empty()) {
             MRB_HIP(hipMalloc(&L->d_gmap_in, sizeof(GhostPair) * grouped.size()));
@@ -2004,7 +2010,7 @@ static int fab_single_step(mrb_level *L, bool last, hipStream_t s)
         if ((rc = mrb_physbc(L, l, s))) return rc;
     if ((rc = fab_batched_step(L, nullptr, last ? 1 : 0, s))) return rc;
     if (!last) {
-        if ((rc = fab_fill_inward(L, s))) return rc;
+        if ((rc = fab_fill_inward(L, L->d_gmap_in, L->d_gmap_in_group, L->n_gmap_in, s))) return rc;
         L->inward_fresh = true;  // (until the next step of the same call)
     }
     return MRB_OK;
