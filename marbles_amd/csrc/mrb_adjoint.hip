@@ -73,13 +73,20 @@ struct IsoArgs {
     double inlet[NQ];
 };
 
+// Blocks take 256 consecutive cells in memory order, so that no lane idles
+// where the rows are no multiple of 64, renumbered to one contiguous run per
+// XCD (xcd_block): the coefficient records, read by 27 neighbours, then come
+// from one L2.
+constexpr int kIsoBlock = 256;
+
 __device__ __forceinline__ bool iso_cell(const IsoArgs &A, int &x, int &y, int &z, int64_t &cell)
 {
-    x = int(blockIdx.x * blockDim.x + threadIdx.x);
-    y = int(blockIdx.y * blockDim.y + threadIdx.y);
-    z = int(blockIdx.z);
-    if (x >= A.nx || y >= A.ny) return false;
-    cell = (int64_t(z) * A.ny + y) * A.nx + x;
+    cell = xcd_block() * kIsoBlock + threadIdx.x;
+    if (cell >= A.N) return false;
+    const uint32_t c = uint32_t(cell), row = c / uint32_t(A.nx);
+    x = int(c - row * uint32_t(A.nx));
+    z = int(row / uint32_t(A.ny));
+    y = int(row - uint32_t(z) * uint32_t(A.ny));
     return true;
 }
 
@@ -221,14 +228,14 @@ __global__ void __launch_bounds__(256) k_iso_loss(const double *__restrict__ f, 
         v = 1e-3 * (0.5 * rho * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]));
         if (x == A.nx - 1) v += u[0] / (double(A.ny) * A.nz);
     }
-    const int t = threadIdx.y * blockDim.x + threadIdx.x;
+    const int t = threadIdx.x;
     sh[t] = v;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
         if (t < w) sh[t] += sh[t + w];
         __syncthreads();
     }
-    if (t == 0) part[(int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = sh[0];
+    if (t == 0) part[xcd_block()] = sh[0];
 }
 
 // lambda_N = dJ/df_N
@@ -404,14 +411,14 @@ __global__ void __launch_bounds__(256) k_iso_adj(
         bu[cell] = base;
         dns[cell] += gns;
     }
-    const int t = threadIdx.y * blockDim.x + threadIdx.x;
+    const int t = threadIdx.x;
     sh[t] = gw;
     __syncthreads();
     for (int s2 = 128; s2 > 0; s2 >>= 1) {
         if (t < s2) sh[t] += sh[t + s2];
         __syncthreads();
     }
-    if (t == 0) part[(int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] += sh[0];
+    if (t == 0) part[xcd_block()] += sh[0];
 }
 
 // transpose of dQ (a 3-point gather of dqbar along each axis) and of
@@ -494,20 +501,20 @@ IsoArgs iso_args(const mrb_iso *S, double tau)
     return A;
 }
 
-dim3 iso_grid(const IsoArgs &A) { return dim3(unsigned((A.nx + 63) / 64), unsigned((A.ny + 3) / 4), unsigned(A.nz)); }
+dim3 iso_grid(const IsoArgs &A) { return dim3(unsigned((A.N + kIsoBlock - 1) / kIsoBlock)); }
 
 int iso_step(const mrb_iso *S, const IsoArgs &A, const double *f, double *fo, const double *ns, hipStream_t s)
 {
-    k_iso_q<<<iso_grid(A), dim3(64, 4, 1), 0, s>>>(f, S->q, A);
+    k_iso_q<<<iso_grid(A), dim3(kIsoBlock), 0, s>>>(f, S->q, A);
     MRB_HIP(hipGetLastError());
-    k_iso_step<<<iso_grid(A), dim3(64, 4, 1), 0, s>>>(f, fo, S->q, ns, A);
+    k_iso_step<<<iso_grid(A), dim3(kIsoBlock), 0, s>>>(f, fo, S->q, ns, A);
     MRB_HIP(hipGetLastError());
     return MRB_OK;
 }
 
 int iso_loss(const mrb_iso *S, const IsoArgs &A, const double *f, hipStream_t s, double *J)
 {
-    k_iso_loss<<<iso_grid(A), dim3(64, 4, 1), 0, s>>>(f, S->part, A);
+    k_iso_loss<<<iso_grid(A), dim3(kIsoBlock), 0, s>>>(f, S->part, A);
     MRB_HIP(hipGetLastError());
     std::vector<double> h(size_t(S->nparts));
     MRB_HIP(hipMemcpyAsync(h.data(), S->part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, s));
@@ -556,8 +563,8 @@ int mrb_iso_create(const int ncell[3], double T0, double rho0, double u_in, mrb_
         A.nx = S->n[0];
         A.ny = S->n[1];
         A.nz = S->n[2];
-        const dim3 g = iso_grid(A);
-        S->nparts = int64_t(g.x) * g.y * g.z;
+        A.N = S->N;
+        S->nparts = int64_t(iso_grid(A).x);
     }
     MRB_HIP(hipMalloc(&S->part, sizeof(double) * size_t(S->nparts)));
     *out = S.release();
@@ -617,7 +624,7 @@ int mrb_iso_forward(mrb_iso *S, const double *ns, double tau, const double *u0, 
     hipStream_t s = as_stream(stream);
     S->rec_valid = false;  // the ping-pong pair holds the recording's final state
     const IsoArgs A = iso_args(S, tau);
-    k_iso_init<<<iso_grid(A), dim3(64, 4, 1), 0, s>>>(S->f[0], u0, A, S->rho0);
+    k_iso_init<<<iso_grid(A), dim3(kIsoBlock), 0, s>>>(S->f[0], u0, A, S->rho0);
     MRB_HIP(hipGetLastError());
     int cur = 0;
     for (int n = 0; n < nsteps; ++n) {
@@ -668,7 +675,7 @@ int mrb_iso_record(mrb_iso *S, const double *ns, double tau, const double *u0, i
     hipStream_t s = as_stream(stream);
     const IsoArgs A = iso_args(S, tau);
     const dim3 g = iso_grid(A);
-    const dim3 b(64, 4, 1);
+    const dim3 b(kIsoBlock);
     const int nseg = (nsteps + every - 1) / every;
     const int last0 = (nseg - 1) * every;  // first step of the last segment
     {
@@ -715,7 +722,7 @@ int mrb_iso_reverse(mrb_iso *S, double *dtau, double *dns, double *du0, void *st
     const double *ns = S->rec_ns, *u0 = S->rec_u0;
     const IsoArgs A = iso_args(S, tau);
     const dim3 g = iso_grid(A);
-    const dim3 b(64, 4, 1);
+    const dim3 b(kIsoBlock);
     const int nseg = (nsteps + every - 1) / every;
     auto state = [&](int sg, int i) { return i == 0 ? S->ckpt[size_t(sg)] : S->seg[size_t(i - 1)]; };
     // reverse sweep: two passes per step
