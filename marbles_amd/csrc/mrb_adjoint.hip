@@ -73,11 +73,11 @@ struct IsoArgs {
     double inlet[NQ];
 };
 
-// Blocks take 256 consecutive cells in memory order, so that no lane idles
+// Blocks take kIsoBlock consecutive cells in memory order, so that no lane idles
 // where the rows are no multiple of 64, renumbered to one contiguous run per
 // XCD (xcd_block): the coefficient records, read by 27 neighbours, then come
 // from one L2.
-constexpr int kIsoBlock = 256;
+constexpr int kIsoBlock = 128;
 
 __device__ __forceinline__ bool iso_cell(const IsoArgs &A, int &x, int &y, int &z, int64_t &cell)
 {
@@ -167,7 +167,7 @@ __device__ __forceinline__ double iso_feq(double rho, const double u[3], const d
     return ((rho * iso_phi(ev(q, 0), u[0], P[0])) * iso_phi(ev(q, 1), u[1], P[1])) * iso_phi(ev(q, 2), u[2], P[2]);
 }
 
-__global__ void __launch_bounds__(256) k_iso_init(double *__restrict__ f, const double *__restrict__ u0, IsoArgs A,
+__global__ void __launch_bounds__(kIsoBlock) k_iso_init(double *__restrict__ f, const double *__restrict__ u0, IsoArgs A,
                                                   double rho0)
 {
     int x, y, z;
@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(256) k_iso_init(double *__restrict__ f, const 
     });
 }
 
-__global__ void __launch_bounds__(256) k_iso_q(const double *__restrict__ f, double *__restrict__ Q, IsoArgs A)
+__global__ void __launch_bounds__(kIsoBlock) k_iso_q(const double *__restrict__ f, double *__restrict__ Q, IsoArgs A)
 {
     int x, y, z;
     int64_t cell;
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(256) k_iso_q(const double *__restrict__ f, dou
     for (int a = 0; a < 3; ++a) Q[a * A.N + cell] = rho * u[a] * (A.k - u[a] * u[a]);
 }
 
-__global__ void __launch_bounds__(256) k_iso_step(const double *__restrict__ f, double *__restrict__ fo,
+__global__ void __launch_bounds__(kIsoBlock) k_iso_step(const double *__restrict__ f, double *__restrict__ fo,
                                                   const double *__restrict__ Q, const double *__restrict__ ns,
                                                   IsoArgs A)
 {
@@ -215,9 +215,9 @@ __global__ void __launch_bounds__(256) k_iso_step(const double *__restrict__ f, 
 }
 
 // J partial sums: outlet-plane u_x / (ny nz) + 1e-3 rho |u|^2 / 2
-__global__ void __launch_bounds__(256) k_iso_loss(const double *__restrict__ f, double *__restrict__ part, IsoArgs A)
+__global__ void __launch_bounds__(kIsoBlock) k_iso_loss(const double *__restrict__ f, double *__restrict__ part, IsoArgs A)
 {
-    __shared__ double sh[256];
+    __shared__ double sh[kIsoBlock];
     int x, y, z;
     int64_t cell;
     double v = 0.0;
@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(256) k_iso_loss(const double *__restrict__ f, 
     const int t = threadIdx.x;
     sh[t] = v;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
+    for (int w = kIsoBlock / 2; w > 0; w >>= 1) {
         if (t < w) sh[t] += sh[t + w];
         __syncthreads();
     }
@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(256) k_iso_loss(const double *__restrict__ f, 
 }
 
 // lambda_N = dJ/df_N
-__global__ void __launch_bounds__(256) k_iso_seed(const double *__restrict__ f, double *__restrict__ lam, IsoArgs A)
+__global__ void __launch_bounds__(kIsoBlock) k_iso_seed(const double *__restrict__ f, double *__restrict__ lam, IsoArgs A)
 {
     int x, y, z;
     int64_t cell;
@@ -277,6 +277,73 @@ __device__ __forceinline__ double lam_at(const double *__restrict__ lams, const 
         if constexpr (ev(q, a) == -1) v -= r[a + 1];
     });
     return v;
+}
+
+// The coefficient records of one block: for each of the nine rows (c_y, c_z)
+// around the block's cells, the row's cells at the block's x, with the cell
+// before the first and the one after the last thread's.  A thread's x
+// neighbours lie in the entries beside its own wherever they lie inside the
+// domain: consecutive threads are consecutive cells.
+struct IsoRecords {
+    double2 r[9][2][kIsoBlock + 2];
+};
+
+template <int cy, int cz>
+constexpr int iso_row = (cz + 1) * 3 + cy + 1;
+
+__device__ __forceinline__ void iso_records(IsoRecords &R, const double *__restrict__ ab, const IsoArgs &A, int x,
+                                            int y, int z)
+{
+    const uint32_t nxy = uint32_t(A.nx) * uint32_t(A.ny);
+    const uint32_t yo[3] = {uint32_t(wrap(y - 1, A.ny)) * uint32_t(A.nx), uint32_t(y) * uint32_t(A.nx),
+                            uint32_t(wrap(y + 1, A.ny)) * uint32_t(A.nx)};
+    const uint32_t zo[3] = {uint32_t(wrap(z - 1, A.nz)) * nxy, uint32_t(z) * nxy, uint32_t(wrap(z + 1, A.nz)) * nxy};
+    const int t = threadIdx.x;
+    const double2 *r = reinterpret_cast<const double2 *>(ab);
+    auto put = [&](int e, uint32_t xe) {
+        static_for<9>([&](auto rc) {
+            constexpr int row = decltype(rc)::value;
+            const int64_t c = 2 * int64_t(zo[row / 3] + yo[row % 3] + xe);
+            R.r[row][0][e] = r[c];
+            R.r[row][1][e] = r[c + 1];
+        });
+    };
+    put(t + 1, uint32_t(x));
+    if (t == 0 && x > 0) put(0, uint32_t(x - 1));
+    if (t == kIsoBlock - 1 && x + 1 < A.nx) put(kIsoBlock + 1, uint32_t(x + 1));
+}
+
+// lam_at and gather_one with the coefficients from R; entries beyond the
+// domain in x are read and not used
+template <int q>
+__device__ __forceinline__ double gather_rec(const double *__restrict__ lams, const IsoRecords &R, const IsoArgs &A,
+                                             int x, int y, int z)
+{
+    constexpr int cx = ev(q, 0), cy = ev(q, 1), cz = ev(q, 2), row = iso_row<cy, cz>;
+    const int ty = wrap(y + cy, A.ny), tz = wrap(z + cz, A.nz);
+    const int tx = x + cx;
+    const bool in = tx >= 0 && tx < A.nx;
+    const double *lq = lams + int64_t(q) * A.N + (int64_t(tz) * A.ny + ty) * A.nx;
+    auto at = [&](int xl, int e) {
+        const double2 r0 = R.r[row][0][e];
+        double v = lq[xl] + r0.x;
+        if constexpr (cx == 1) v += r0.y;
+        if constexpr (cx == -1) v -= r0.y;
+        if constexpr (cy != 0 || cz != 0) {
+            const double2 r1 = R.r[row][1][e];
+            if constexpr (cy == 1) v += r1.x;
+            if constexpr (cy == -1) v -= r1.x;
+            if constexpr (cz == 1) v += r1.y;
+            if constexpr (cz == -1) v -= r1.y;
+        }
+        return v;
+    };
+    const int e = int(threadIdx.x) + 1;
+    const double v = at(tx < 0 ? 0 : (tx >= A.nx ? A.nx - 1 : tx), e + cx);
+    double l = in ? v : 0.0;
+    if constexpr (cx == -1)
+        if (x == A.nx - 1) l += at(x, e);
+    return l;
 }
 
 // transpose of the pull, as a gather: f_q(x) was read by the cell x + c_q
@@ -317,20 +384,33 @@ __device__ __forceinline__ void iso_gather_lambda(const double *__restrict__ lam
 // in bu (base, ms ubar / rho), together with dJ/d(dQ) times dt w_corr
 // (dqbar) and u of the pulled state (uo); dJ/dn_s is accumulated and dJ/dw
 // summed per block.
+// Bound by the 27 + 27 population reads and 27 writes plus the issue of the
+// neighbours' coefficients: 51 two-word reads of 32-byte records per cell,
+// from LDS (IsoRecords: 18 global reads per cell), behind the pull's loads.
+// 96x80x64: 130 us with 64 x 4 blocks, 123 with consecutive cells and global
+// records, 106 with records in LDS; 77 without any gather (last step).
+// kIsoBlock 128: four blocks of 38 KB share a CU at two waves per SIMD.
 template <bool GATHER>
-__global__ void __launch_bounds__(256) k_iso_adj(
+__global__ void __launch_bounds__(kIsoBlock) k_iso_adj(
     const double *__restrict__ f, const double *__restrict__ Q, const double *__restrict__ lin,
     const double *__restrict__ ab, const double *__restrict__ ns, double *__restrict__ lams,
     double *__restrict__ dqbar, double *__restrict__ uo, double *__restrict__ bu, double *__restrict__ dns,
     double *__restrict__ part, IsoArgs A)
 {
-    __shared__ double sh[256];
+    __shared__ double sh[kIsoBlock];
+    __shared__ std::conditional_t<GATHER, IsoRecords, char> rec;
     int x, y, z;
     int64_t cell;
     double gw = 0.0;
-    if (iso_cell(A, x, y, z, cell)) {
-        double fs[NQ], rho, u[3], dq[3];
+    const bool own = iso_cell(A, x, y, z, cell);
+    double fs[NQ];
+    if (own) {
         iso_pull(f, A, x, y, z, fs);
+        if constexpr (GATHER) iso_records(rec, ab, A, x, y, z);
+    }
+    if constexpr (GATHER) __syncthreads();
+    if (own) {
+        double rho, u[3], dq[3];
         iso_moments(fs, A, rho, u);
         iso_dq(Q, A, x, y, z, cell, dq);
         const double w = A.w;
@@ -372,7 +452,7 @@ __global__ void __launch_bounds__(256) k_iso_adj(
         auto lam_in = [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             if constexpr (GATHER)
-                return gather_one<q>(lin, ab, A, x, y, z);
+                return gather_rec<q>(lin, rec, A, x, y, z);
             else
                 return lin[int64_t(q) * A.N + cell];
         };
@@ -414,7 +494,7 @@ __global__ void __launch_bounds__(256) k_iso_adj(
     const int t = threadIdx.x;
     sh[t] = gw;
     __syncthreads();
-    for (int s2 = 128; s2 > 0; s2 >>= 1) {
+    for (int s2 = kIsoBlock / 2; s2 > 0; s2 >>= 1) {
         if (t < s2) sh[t] += sh[t + s2];
         __syncthreads();
     }
@@ -428,7 +508,7 @@ __global__ void __launch_bounds__(256) k_iso_adj(
 // pulled population's lambda, alpha + beta . c_q, with alpha = base +
 // sum_a Qbar_a 2 u_a^3 and beta_a = ms ubar_a / rho + Qbar_a (k - 3 u_a^2) ms
 // (base and ms ubar / rho from bu).
-__global__ void __launch_bounds__(256) k_iso_adj_q(const double *__restrict__ dqbar, const double *__restrict__ uo,
+__global__ void __launch_bounds__(kIsoBlock) k_iso_adj_q(const double *__restrict__ dqbar, const double *__restrict__ uo,
                                                    const double *__restrict__ bu, double *__restrict__ ab, IsoArgs A)
 {
     int x, y, z;
@@ -459,7 +539,7 @@ __global__ void __launch_bounds__(256) k_iso_adj_q(const double *__restrict__ dq
 }
 
 // dJ/du0 from lambda_0 (gathered) through the initial equilibrium
-__global__ void __launch_bounds__(256) k_iso_u0grad(const double *__restrict__ lams, const double *__restrict__ ab,
+__global__ void __launch_bounds__(kIsoBlock) k_iso_u0grad(const double *__restrict__ lams, const double *__restrict__ ab,
                                                     const double *__restrict__ u0, double *__restrict__ du0, IsoArgs A,
                                                     double rho0)
 {
@@ -519,9 +599,9 @@ int iso_loss(const mrb_iso *S, const IsoArgs &A, const double *f, hipStream_t s,
     std::vector<double> h(size_t(S->nparts));
     MRB_HIP(hipMemcpyAsync(h.data(), S->part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, s));
     MRB_HIP(hipStreamSynchronize(s));
-    double acc = 0.0;
+    long double acc = 0.0L;  // thousands of block sums: in double their rounding exceeds the tree sums' own
     for (double v : h) acc += v;
-    *J = acc;
+    *J = double(acc);
     return MRB_OK;
 }
 
@@ -769,9 +849,9 @@ int mrb_iso_reverse(mrb_iso *S, double *dtau, double *dns, double *du0, void *st
     std::vector<double> part(size_t(S->nparts));
     MRB_HIP(hipMemcpyAsync(part.data(), S->part, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
     MRB_HIP(hipStreamSynchronize(s));
-    double gw = 0.0;
+    long double gw = 0.0L;
     for (double v : part) gw += v;
-    *dtau = gw * (-1.0 / (tau * tau));  // w = 1/tau
+    *dtau = double(gw) * (-1.0 / (tau * tau));  // w = 1/tau
     return MRB_OK;
 }
 
