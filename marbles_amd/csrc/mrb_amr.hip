@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(kAmrBlock) k_coalesce(
 // Coarse-to-fine interpolation of FillPatchTwoLevels / InterpFromCoarseLevel
 // with amrex::cell_cons_interp (FillPatchOps.H:124-128,174-177,190): AMReX's
 // conservative linear scheme without linear limiting, ratio 2.  Per coarse
-// parent and component (k_explode_slopes): monotonised-central slopes, the
+// parent and component (parent_slopes): monotonised-central slopes, the
 // centred difference replaced at an ext_dir face (every non-periodic face,
 // LBM.cpp:108-150) by the one-sided second-order form through the value
 // beyond the face; then one factor alpha <= 1 so that no child leaves the
@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(kAmrBlock) k_coalesce(
 // from holds -1 beyond a non-periodic face: BCFill only writes the boundary
 // value where iv + c_q lies inside the patch shrunk by the level's 3 ghost
 // cells (BC.H:375-380), which a ghost's neighbour never does.  Per child
-// (k_explode): ((c + o_x s_x) + o_y s_y) + o_z s_z with o = -+1/4.
+// (k_explode, k_explode_groups): ((c + o_x s_x) + o_y s_y) + o_z s_z with o = -+1/4.
 // Every load is issued unconditionally: the fab's ghost layers (ng >= 2,
 // checked when the map is built) hold P +- 2 in every direction.
 // the coarse value and the limited slopes of one component of the parent at c
