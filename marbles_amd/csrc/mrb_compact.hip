@@ -1142,7 +1142,8 @@ __host__ __device__ __forceinline__ int64_t domain_cells(const CompactArgs &A)
 // blocks' lanes), XCD: one contiguous run of blocks per XCD for the kernels
 // that read face neighbours.  200x160x144, FP64: k_macro 442 -> 429 us (with
 // f and g of a cell in one load; 436 in XCD runs: nothing is shared),
-// k_vorticity 97 -> 80 us, k_tag 14 -> 11 us.
+// k_vorticity 97 -> 80 us, k_tag 14 -> 11 us.  256^3, FP16: k_macro 720 ->
+// 484 us (one 4-byte load for two of 2).
 template <bool XCD = true>
 __device__ __forceinline__ bool cell_flat(const CompactArgs &A, int &x, int &y, int &z, int64_t &cell)
 {
