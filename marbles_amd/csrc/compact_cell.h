@@ -248,9 +248,10 @@ constexpr int qwith(int d, int c, int k)
 // a Channel or Parabolic inlet profile, PRESSURE faces
 constexpr int kBcxProfile = 1;
 constexpr int kBcxPressure = 2;
-// the profile inlet's only VELOCITY face is x-lo, as in the cylinder and duct
-// decks: the lookups of the other faces, merged into one pull, take the FP64
-// kernels from 145 and 201 registers to 256
+// the profile inlet's only VELOCITY face is x-lo, as in the channel and duct
+// workloads and the 660x123x4 cylinder deck: the lookups of the other faces,
+// merged into one pull, take the FP64 passes from 150 and 200 registers to 228
+// and 239.  (The 246x576x4 deck's inlet at y-lo takes them: 141 us per step.)
 constexpr int kBcxProfileX = 4;
 
 // pressure_bc_f (BC.H:222-271) for the fluid cell (x, y, z) next to a
@@ -470,8 +471,12 @@ __device__ __forceinline__ PullBits pull_raw(
 // The loads of the pull before the cell's stream mask is known: every source
 // read as if it were fluid (clamped into the domain beyond a non-periodic
 // face), in one fixed sequence without a branch.  pull_settle, given the
-// mask, keeps them when every source of the wave is read directly and
-// repeats the pull on the general path otherwise.
+// mask, keeps them where the source is read directly and loads the others
+// (walls, solid sources) again, lane by lane.  Repeating the whole pull of a wave
+// with one such source took more than the mask's latency had cost: 96x64x48
+// cells between six walls, FP64, 101 us per step against 86 (88 on row blocks,
+// whose pull waits for the mask); 160x120x100 with a pressure outlet, whose
+// ghosts need no second load, 510 against 404.
 template <class T, bool NT>
 __device__ __forceinline__ void pull_ahead(const T *__restrict__ f, const CompactArgs &A, int x, int y, int z,
                                            T rf[NQ], T rg[NQ])
@@ -499,6 +504,31 @@ __device__ __forceinline__ void pull_ahead(const T *__restrict__ f, const Compac
         load_stored_pair<NT>(reinterpret_cast<const T *>(b + (yo[cy + 1] + xo[cx + 1])), rf[q], rg[q]);
     });
 }
+// The element that direction q's source is read from when it is a wall's ghost or
+// a solid cell, as pull_raw's general path resolves it (kept apart from it: the
+// z-sweep on FP32 storage lost 10 % when it took its elements from here).  pz:
+// the cell read was moved inward across a z OUTFLOW face.
+template <int q, class T>
+__device__ __forceinline__ int64_t wall_e(const CompactArgs &A, const bool gx[3], const bool gy[3], const bool gz[3],
+                                          int64_t cell, bool &pz)
+{
+    constexpr int cx = ev(q, 0), cy = ev(q, 1), cz = ev(q, 2);
+    const bool hx = gx[cx + 1], hy = gy[cy + 1], hz = gz[cz + 1];
+    const uint32_t tfz = (A.bcpack >> (4 * (cz > 0 ? 2 : 5))) & 15u;
+    const uint32_t tfy = (A.bcpack >> (4 * (cy > 0 ? 1 : 4))) & 15u;
+    const uint32_t tfx = (A.bcpack >> (4 * (cx > 0 ? 0 : 3))) & 15u;
+    pz = hz && tfz == MRB_BC_OUTFLOW;
+    const bool py = hy && tfy == MRB_BC_OUTFLOW && (pz || !hz);
+    const bool px = hx && tfx == MRB_BC_OUTFLOW && (py || !hy) && (pz || !hz);
+    const uint32_t t = (hz && !pz) ? tfz : (hy && !py) ? tfy : (hx && !px) ? tfx : uint32_t(MRB_BC_OUTFLOW);
+    const int32_t roff = (pz ? cz * A.nx * A.ny : 0) + (py ? cy * A.nx : 0) + (px ? cx : 0);
+    int comp = kBounce[q];
+    comp = t == MRB_BC_SLIPX ? reflect(q, 0) : comp;
+    comp = t == MRB_BC_SLIPY ? reflect(q, 1) : comp;
+    comp = t == MRB_BC_SLIPZ ? reflect(q, 2) : comp;
+    return int64_t(comp) * A.cs + int64_t(uint32_t(int32_t(uint32_t(cell)) + roff)) * kCellStride<T>;
+}
+
 template <int BCX, class T, bool NT>
 __device__ __forceinline__ PullBits pull_settle(const T *__restrict__ f, const CompactArgs &A, int x, int y, int z,
                                                 int64_t cell, uint32_t mask, T rf[NQ], T rg[NQ])
@@ -515,8 +545,46 @@ __device__ __forceinline__ PullBits pull_settle(const T *__restrict__ f, const C
         targets3(z, A.nz, A.per[2], tz, gz);
         const SourceSets S = source_sets<BCX>(A, gx, gy, gz);
         pb.cmask = S.V;
-        if (__any(S.nondirect(mask) != 0u))
-            pb = pull_raw<BCX, T, false, NT>(f, A, x, y, z, cell, mask, rf, rg);
+        pb.Pm = S.Pm;
+        // (a PRESSURE ghost's value replaces what was loaded)
+        const uint32_t nd = S.nondirect(mask) & ~S.Pm;
+        pb.dmask = kAllQ & ~nd;
+        if (__any(nd != 0u)) {
+            // An FP32 pair is kept as one word meanwhile: as two values the
+            // compiler may copy each pair behind its load, which then waits
+            // for it (pass 2 of a y-lo profile inlet, 246x576x4: 98 us per step
+            // against 88); of an FP16 pair the word costs more scratch
+            struct Pair {
+                T f, g;
+            };
+            using Bits = std::conditional_t<std::is_same<T, float>::value, uint64_t, Pair>;
+            constexpr bool kWord = std::is_same<T, float>::value;
+            Bits word[NQ];
+            if constexpr (kWord)
+                for (int q = 0; q < NQ; ++q) word[q] = __builtin_bit_cast(Bits, Pair{rf[q], rg[q]});
+            static_for<NQ>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                if ((nd >> q) & 1u) {
+                    bool pz;
+                    Pair v;
+                    load_stored_pair<NT>(f + wall_e<q, T>(A, gx, gy, gz, cell, pz), v.f, v.g);
+                    pb.zmove |= uint32_t(pz) << q;
+                    if constexpr (kWord) {
+                        word[q] = __builtin_bit_cast(Bits, v);
+                    } else {
+                        rf[q] = v.f;
+                        rg[q] = v.g;
+                    }
+                }
+            });
+            if constexpr (kWord)
+                for (int q = 0; q < NQ; ++q) {
+                    asm volatile("" : "+v"(word[q]));
+                    const Pair v = __builtin_bit_cast(Pair, word[q]);
+                    rf[q] = v.f;
+                    rg[q] = v.g;
+                }
+        }
     }
     return pb;
 }

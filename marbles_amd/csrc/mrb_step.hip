@@ -4,8 +4,8 @@
 // the row length: on 301-cell rows 256x1 blocks leave 41 % of their lanes
 // idle, on 24-cell rows 91 %.  A tile's z is the same for all its lanes, so
 // the pull's loads take a scalar base and a 32-bit offset, and they are
-// issued together with the load of the stream mask: the few waves next to
-// solid cells or walls repeat them on the general path.
+// issued together with the load of the stream mask: lanes next to solid cells
+// or walls load those sources again (pull_settle).
 //
 // k_step: both passes of an FP64 level in one launch.  Pass 1 (Q_corr of the
 // post-stream state) and pass 2 (collide, which needs the six face
