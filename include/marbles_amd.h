@@ -210,7 +210,7 @@ int mrb_advance_timed(mrb_level *lvl, int nsteps, void *stream, double *kernel_m
  *   7  the two-pass step on tiles of 256 (shifted FP32: 128) consecutive
  *      cells of a z-plane; FP64 levels of 2^18 cells and more run both
  *      passes in one launch (mrb_advance_timed: its time in slot 0);
- *   8  the same as 5;
+ *   8  the passes of 5 on 256x1-cell row blocks;
  *   9  shifted FP32 storage only, no PRESSURE faces: the collide pass in
  *      FP32 arithmetic on the stored deviations from the rest state (FP64
  *      moments and equilibrium coefficients; mass and energy residuals on

@@ -776,11 +776,10 @@ static int two_pass_tp(mrb_level *L, int variant, hipStream_t s, hipEvent_t *ev)
     const T *g = (const T *)L->pop[1][L->cur];
     T *fo = (T *)L->pop[0][1 - L->cur];
     T *go = (T *)L->pop[1][1 - L->cur];
-    if (variant == kX256Variant || variant == kF32X256Variant || variant == kHalf32Variant ||
-        variant == kHalf32X256Variant) {
+    if (variant == kX256Variant || variant == kF32X256Variant || variant == kHalf32Variant) {
         if (variant == kF32X256Variant && !std::is_same<T, float>::value)
             return set_error(MRB_E_UNSUPPORTED, "k_collide_f32: shifted FP32 storage without PRESSURE faces only");
-        if ((variant == kHalf32Variant || variant == kHalf32X256Variant) && !kIsHalf<T>)
+        if (variant == kHalf32Variant && !kIsHalf<T>)
             return set_error(MRB_E_UNSUPPORTED, "k_collide_h32: scaled FP16 storage without PRESSURE faces only");
         if (tile_step_fits(L)) return compact_tile_step(L, variant != kX256Variant, s, ev);
         // planes past the tiles' 32-bit offsets: the same arithmetic on blocks
@@ -912,14 +911,17 @@ static int two_pass_tp(mrb_level *L, int variant, hipStream_t s, hipEvent_t *ev)
                              "k_collide_f32: shifted FP32 storage without PRESSURE faces only");
         }
     }
-    if (variant == kHalf32Variant) {
+    if (variant == kHalf32Variant || variant == kHalf32X256Variant) {
         if constexpr (kIsHalf<T> && (BCX & kBcxPressure) == 0) {
+            // 256x1 blocks, or (planes past the tiles' offsets) 64x4
+            const bool x256 = variant == kHalf32X256Variant;
+            const dim3 grid = x256 ? grid_of(A, 1, 256) : grid_of(A), block = x256 ? dim3(256, 1, 1) : dim3(64, 4, 1);
             if (ev) MRB_HIP(hipEventRecord(ev[0], s));
-            k_qpass<T, BCX><<<grid_of(A), dim3(64, 4, 1), 0, s>>>(f, g, L->d_mask, L->d_q, A, L->bcdev, sh, h16, L->cp);
+            k_qpass<T, BCX><<<grid, block, 0, s>>>(f, g, L->d_mask, L->d_q, A, L->bcdev, sh, h16, L->cp);
             MRB_HIP(hipGetLastError());
             if (ev) MRB_HIP(hipEventRecord(ev[1], s));
-            k_collide_h32<T, BCX><<<grid_of(A), dim3(64, 4, 1), 0, s>>>(f, g, fo, go, L->d_mask, L->d_q, A, L->bcdev,
-                                                                         sh, h16, L->cp);
+            k_collide_h32<T, BCX><<<grid, block, 0, s>>>(f, g, fo, go, L->d_mask, L->d_q, A, L->bcdev, sh, h16,
+                                                         L->cp);
             MRB_HIP(hipGetLastError());
             if (ev) MRB_HIP(hipEventRecord(ev[2], s));
             return MRB_OK;

@@ -407,7 +407,7 @@ constexpr int kRows2Variant = 4;  // two passes on 64x2 blocks
 constexpr int kHalf32Variant = 5; // scaled FP16 storage, FP32 arithmetic in pass 2, tiles of consecutive cells
 constexpr int kX128Variant = 6;   // two passes on 128x2 blocks
 constexpr int kX256Variant = 7;   // two passes on tiles of consecutive cells (mrb_step.hip)
-constexpr int kHalf32X256Variant = 8; // the same as 5
+constexpr int kHalf32X256Variant = 8; // the passes of 5 on 256x1 row blocks
 constexpr int kF32Variant = 9;         // shifted FP32 storage, FP32 arithmetic in pass 2 (64x2 blocks)
 constexpr int kF32X256Variant = 10;    // variant 9 on tiles of consecutive cells
 constexpr int kSweepVariant = 11;      // single-pass z-sweep, one block per x-row (FP64 / FP32, rows <= 256 cells)
@@ -415,8 +415,8 @@ constexpr int kSweepRingPlanes = 8;    // planes of Q_y the z-sweep keeps for th
 constexpr int kSweepX64Variant = 12;   // the z-sweep on single-wave blocks of 64 cells of a row (FP64)
 constexpr int kSweepF32Variant = 13;   // the z-sweep with the FP32-arithmetic collide (shifted FP32)
 // the variants whose pass 2 computes in FP32 (their results differ from the
-// FP64-arithmetic variants'), and the FP64-arithmetic variant with the same
-// block shape that replaces one on a level with PRESSURE faces
+// FP64-arithmetic variants'), and the FP64-arithmetic variant that replaces one
+// on a level with PRESSURE faces
 inline bool fp32_collide_variant(int v)
 {
     return v == kHalf32Variant || v == kHalf32X256Variant || v == kF32Variant || v == kF32X256Variant ||

@@ -68,6 +68,23 @@ def test_fp32_arithmetic_tile_step_equals_row_blocks_at_boundaries(engine, case)
         assert np.isfinite(a).all() and np.array_equal(a, b), case
 
 
+@pytest.mark.parametrize("case", ["walls", "open_corners", "duct", "y_inlet"])
+def test_fp16_default_step_equals_row_blocks_at_boundaries(engine, case):
+    """The scaled FP16 storage's default step (FP32 arithmetic in pass 2 on
+    tiles): the row-block variant launches its own kernel, with the same scales
+    and box maxima."""
+    out = []
+    for variant in (None, "k_qpass_x256+k_collide_h32_x256"):
+        E = configs.build_level(CASES[case]((37, 19, 14)), layout="compact", storage="f16s")
+        if variant:
+            E.set_hot_kernel(variant)
+        E.advance(12)
+        out.append([E.valid(name) for name in ("f", "g")])
+        E.close()
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b), case
+
+
 def test_full_size_y_inlet_deck_equals_row_blocks(engine):
     """The 246 x 576 x 4 cylinder deck with its parabolic inlet at y-lo."""
     out = []
