@@ -170,7 +170,8 @@ def time_level(lvl, steps: int, warmup: int, profile_steps: int, sh, torch, auto
     torch.cuda.synchronize()
     secs = time.perf_counter() - t0
     prof = lvl.advance_timed(profile_steps, stream=sh)
-    return {"secs": secs, "per_kernel_ms": {k: v / profile_steps for k, v in prof.items()}}
+    return {"secs": secs, "variant": lvl.hot_kernel_name(),
+            "per_kernel_ms": {k: v / profile_steps for k, v in prof.items()}}
 
 
 def run_amr(args, torch) -> int:
@@ -605,7 +606,7 @@ def main() -> int:
                 "max_rel_velocity_error": du,
                 "max_rel_density_error": dr,
                 "compared_after_steps": args.warmup + args.steps + args.profile_steps,
-                "arithmetic": "f32" if any(("_h32" in k or "_f32" in k) for k in rr["per_kernel_ms"]) else "f64",
+                "arithmetic": "f32" if ("_h32" in rr["variant"] or "_f32" in rr["variant"]) else "f64",
                 "bytes_per_update": br,
                 "achieved_gbs": round(br * cells / (kms * 1e-3) / 1e9, 1),
                 "traffic": measured_traffic(st, rr["per_kernel_ms"]) if n == 256 else None,

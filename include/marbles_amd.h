@@ -193,7 +193,7 @@ int mrb_stream_collide(mrb_level *lvl, void *stream);
 int mrb_advance(mrb_level *lvl, int nsteps, void *stream);
 /* nsteps fused steps with HIP events recorded on `stream` around each kernel
  * of the step; kernel_ms[k] receives the summed duration of kernel slot k
- * (slots are named by mrb_hot_kernel_name, separated by '+'), *nslots the
+ * (slots are named by mrb_hot_kernel_launches, separated by '+'), *nslots the
  * number of slots (at most 4).  Synchronous.  Compact layout only. */
 int mrb_advance_timed(mrb_level *lvl, int nsteps, void *stream, double *kernel_ms, int *nslots);
 /* Kernel variants of the compact-layout step.
@@ -209,7 +209,7 @@ int mrb_advance_timed(mrb_level *lvl, int nsteps, void *stream, double *kernel_m
  *   6  the two-pass step on 128x2-cell blocks;
  *   7  the two-pass step on tiles of 256 (shifted FP32: 128) consecutive
  *      cells of a z-plane; FP64 levels of 2^18 cells and more run both
- *      passes in one launch (mrb_advance_timed: its time in slot 0);
+ *      passes in one launch;
  *   8  the passes of 5 on 256x1-cell row blocks;
  *   9  shifted FP32 storage only, no PRESSURE faces: the collide pass in
  *      FP32 arithmetic on the stored deviations from the rest state (FP64
@@ -493,6 +493,10 @@ const char *mrb_last_error(void);
 int mrb_stencil(int evs[81], double weights[27], int bounce_dirs[27]);
 /* Name of the kernel variant used by mrb_stream_collide. */
 const char *mrb_hot_kernel_name(const mrb_level *lvl);
+/* The kernels a step of that variant launches on this level, separated by
+ * '+' (variants 5, 7 and 10 launch the tile kernels or k_step, by storage and
+ * size). */
+const char *mrb_hot_kernel_launches(const mrb_level *lvl);
 /* Device pointers of the current population buffers (for zero-copy use by
  * the Python/torch wrappers).  lattice 0 = f, 1 = g.  Fab layout: each
  * box's FAB, components contiguous.  Compact layout: f_q and g_q of a cell

@@ -121,6 +121,7 @@ SIGNATURES = {
     "mrb_stream_copy": (c_int, [c_void_p, c_void_p, ctypes.c_int64, c_int, c_void_p]),
     "mrb_last_error": (c_char_p, []),
     "mrb_hot_kernel_name": (c_char_p, [c_void_p]),
+    "mrb_hot_kernel_launches": (c_char_p, [c_void_p]),
     "mrb_population_ptr": (c_int, [c_void_p, c_int, POINTER(c_void_p), POINTER(c_int64)]),
     "mrb_storage_saturations": (c_int, [c_void_p, POINTER(c_int64)]),
     "mrb_storage_shift": (c_int, [c_void_p, c_int, POINTER(c_double)]),

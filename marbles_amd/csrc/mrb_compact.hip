@@ -16,6 +16,8 @@
 //              neighbours, equilibria, relax, write 54 populations to B.
 #include "compact_cell.h"
 
+#include <cstring>
+
 namespace mrb {
 namespace {
 
@@ -765,6 +767,13 @@ int compact_build_mask(mrb_level *L, hipStream_t s)
 
 // Two-pass step; reads the current buffers, writes the spare ones, does not
 // flip.  ev (if not null) receives events before, between and after.
+static bool tile_variant(int v) { return v == kX256Variant || v == kF32X256Variant || v == kHalf32Variant; }
+// planes past the tiles' 32-bit offsets: the same arithmetic on blocks
+static int tile_fallback(int v)
+{
+    return v == kX256Variant ? kX128Variant : (v == kF32X256Variant ? kF32Variant : kHalf32Variant);
+}
+
 template <class T, int BCX>
 static int two_pass_tp(mrb_level *L, int variant, hipStream_t s, hipEvent_t *ev)
 {
@@ -776,14 +785,13 @@ static int two_pass_tp(mrb_level *L, int variant, hipStream_t s, hipEvent_t *ev)
     const T *g = (const T *)L->pop[1][L->cur];
     T *fo = (T *)L->pop[0][1 - L->cur];
     T *go = (T *)L->pop[1][1 - L->cur];
-    if (variant == kX256Variant || variant == kF32X256Variant || variant == kHalf32Variant) {
+    if (tile_variant(variant)) {
         if (variant == kF32X256Variant && !std::is_same<T, float>::value)
             return set_error(MRB_E_UNSUPPORTED, "k_collide_f32: shifted FP32 storage without PRESSURE faces only");
         if (variant == kHalf32Variant && !kIsHalf<T>)
             return set_error(MRB_E_UNSUPPORTED, "k_collide_h32: scaled FP16 storage without PRESSURE faces only");
         if (tile_step_fits(L)) return compact_tile_step(L, variant != kX256Variant, s, ev);
-        // planes past the tiles' 32-bit offsets: the same arithmetic on blocks
-        variant = variant == kX256Variant ? kX128Variant : (variant == kF32X256Variant ? kF32Variant : kHalf32Variant);
+        variant = tile_fallback(variant);
     }
     if (variant == kSweepX64Variant) {
         if constexpr (std::is_same<T, double>::value) {
@@ -987,15 +995,19 @@ const char *compact_variant_name(int index)
     return index < kNumTwoPassVariants ? kTwoPassNames[index] : kFusedVariants[index - kNumTwoPassVariants].name;
 }
 
+const char *compact_step_kernels(const mrb_level *L)
+{
+    if (!tile_variant(L->hot)) return compact_variant_name(L->hot);
+    return tile_step_fits(L) ? compact_tile_kernels(L, L->hot != kX256Variant)
+                             : compact_variant_name(tile_fallback(L->hot));
+}
+
 static int step_impl(mrb_level *L, hipStream_t s, bool events, int &nslots)
 {
     int rc;
     if (L->hot < kNumTwoPassVariants) {
         rc = two_pass(L, L->hot, s, events ? L->ev : nullptr);
-        nslots = (L->hot == kOnePassVariant || L->hot == kSweepVariant || L->hot == kSweepX64Variant ||
-                  L->hot == kSweepF32Variant)
-                     ? 1
-                     : 2;
+        nslots = std::strchr(compact_step_kernels(L), '+') ? 2 : 1;
     } else {
         if (events) MRB_HIP(hipEventRecord(L->ev[0], s));
         rc = fused_launch(L, L->hot - kNumTwoPassVariants, s);

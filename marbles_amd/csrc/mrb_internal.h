@@ -391,6 +391,8 @@ int compact_stream_collide_events(mrb_level *L, hipStream_t s, int &nslots);
 int compact_stream_only(mrb_level *L, hipStream_t s);
 int compact_build_mask(mrb_level *L, hipStream_t s);
 const char *compact_kernel_name(const mrb_level *L);
+// the kernels that a step of the level's variant launches, '+' between them
+const char *compact_step_kernels(const mrb_level *L);
 // single-pass kernels (mrb_fused.hip): launch reads the current buffer and
 // writes the spare one; step also flips the buffers
 int fused_launch(mrb_level *L, int variant, hipStream_t s);
@@ -440,6 +442,8 @@ int compact_two_pass_launch(mrb_level *L, int variant, hipStream_t s);
 // current buffers, writes the spare ones, does not flip; ev (if not null)
 // receives events before, between and after the passes
 int compact_tile_step(mrb_level *L, bool fp32_collide, hipStream_t s, hipEvent_t *ev);
+// the kernels it launches, '+' between the passes
+const char *compact_tile_kernels(const mrb_level *L, bool fp32_collide);
 // (32-bit byte offsets within a plane)
 inline bool tile_step_fits(const mrb_level *L) { return int64_t(L->ncell[0]) * L->ncell[1] < (int64_t(1) << 28); }
 inline uint32_t tiles_per_plane(int nx, int ny, int tile)

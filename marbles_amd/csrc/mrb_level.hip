@@ -2401,6 +2401,12 @@ const char *mrb_hot_kernel_name(const mrb_level *L)
     return L->layout == MRB_LAYOUT_COMPACT ? compact_kernel_name(L) : "fab-stages";
 }
 
+const char *mrb_hot_kernel_launches(const mrb_level *L)
+{
+    if (!L) return "";
+    return L->layout == MRB_LAYOUT_COMPACT ? compact_step_kernels(L) : "fab-stages";
+}
+
 int mrb_population_ptr(const mrb_level *L, int lattice, void **dev_ptr, int64_t *bytes)
 {
     if (!L || !dev_ptr || lattice < 0 || lattice > 1) return set_error(MRB_E_ARG, "bad argument");

@@ -362,6 +362,12 @@ __global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) 
                                      TileCell::of<TILE>(blockIdx.x, A, G), ListArgs{}, 0u);
 }
 
+// both passes in one launch
+bool one_launch(const mrb_level *L)
+{
+    return L->storage == MRB_STORAGE_F64 && L->total_cells >= kListCells && L->ncell[0] <= kListRow;
+}
+
 template <class T, int BCX, int ARITH>
 int launch(mrb_level *L, hipStream_t s, hipEvent_t *ev)
 {
@@ -376,15 +382,13 @@ int launch(mrb_level *L, hipStream_t s, hipEvent_t *ev)
     const TileArgs G{nxy, tpp, FastDiv(tpp), FastDiv(uint32_t(A.nx))};
     if (ev) MRB_HIP(hipEventRecord(ev[0], s));
     if constexpr (std::is_same<T, double>::value) {
-        if (L->total_cells >= kListCells && A.nx <= kListRow) {
+        if (one_launch(L)) {
             const uint32_t lag = std::min(ntiles, tpp + 1u + kListAhead);
             const ListArgs S{ntiles, lag, uint32_t(A.nx + kStepTile - 1) / kStepTile, L->d_step_counter,
                              L->d_step_flags};
             k_step<BCX><<<2u * ntiles, kStepTile, 0, s>>>(f, fo, L->d_mask, L->d_q, A, L->bcdev, sh, L->cp, G, S);
             MRB_HIP(hipGetLastError());
-            // one launch: its time in slot 0, slot 1 stays empty
             if (ev) MRB_HIP(hipEventRecord(ev[1], s));
-            if (ev) MRB_HIP(hipEventRecord(ev[2], s));
             return MRB_OK;
         }
     }
@@ -426,6 +430,13 @@ int compact_tile_step(mrb_level *L, bool fp32_collide, hipStream_t s, hipEvent_t
     if (L->storage == MRB_STORAGE_F32_SHIFTED)
         return fp32_collide ? launch_bcx<float, kStepF32Dev>(L, s, ev) : launch_bcx<float, kStepF64>(L, s, ev);
     return fp32_collide ? launch_bcx<_Float16, kStepH32>(L, s, ev) : launch_bcx<_Float16, kStepF64>(L, s, ev);
+}
+
+const char *compact_tile_kernels(const mrb_level *L, bool fp32_collide)
+{
+    if (one_launch(L)) return "k_step";
+    return fp32_collide && L->storage == MRB_STORAGE_F16_SCALED ? "k_qpass_tile+k_collide_tile_w4"
+                                                                : "k_qpass_tile+k_collide_tile";
 }
 
 }  // namespace mrb

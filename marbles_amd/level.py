@@ -221,7 +221,7 @@ class Level:
         ms = (c_double * 4)()
         ns = c_int()
         check(self.lib.mrb_advance_timed(self.h, int(nsteps), stream, ms, ctypes.byref(ns)))
-        names = self.hot_kernel_name().split("+")
+        names = self.hot_kernel_launches().split("+")
         return {names[k] if k < len(names) else f"k{k}": ms[k] for k in range(ns.value)}
 
     @staticmethod
@@ -335,6 +335,10 @@ class Level:
 
     def hot_kernel_name(self) -> str:
         return self.lib.mrb_hot_kernel_name(self.h).decode()
+
+    def hot_kernel_launches(self) -> str:
+        """The kernels a step launches, '+' between them."""
+        return self.lib.mrb_hot_kernel_launches(self.h).decode()
 
     def population_ptr(self, lattice: int) -> tuple[int, int]:
         p = c_void_p()

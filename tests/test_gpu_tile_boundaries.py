@@ -96,3 +96,22 @@ def test_full_size_y_inlet_deck_equals_row_blocks(engine):
         E.close()
     for a, b in zip(*out):
         assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage,shape,variant,launches", [
+    ("f64", (37, 19, 14), None, "k_qpass_tile+k_collide_tile"),
+    ("f64", (131, 47, 45), None, "k_step"),
+    ("f64", (131, 47, 45), "k_qpass_x128+k_collide_x128", "k_qpass_x128+k_collide_x128"),
+    ("f32s", (131, 47, 45), None, "k_qpass_tile+k_collide_tile"),
+    ("f16s", (131, 47, 45), None, "k_qpass_tile+k_collide_tile_w4"),
+    ("f16s", (37, 19, 14), "k_qpass_x256+k_collide_h32_x256", "k_qpass_x256+k_collide_h32_x256"),
+])
+def test_timed_steps_name_the_kernels_that_run(engine, storage, shape, variant, launches):
+    """One slot per launched kernel, under its own name, each with a time."""
+    E = configs.build_level(CASES["walls"](shape), layout="compact", storage=storage)
+    if variant:
+        E.set_hot_kernel(variant)
+    assert E.hot_kernel_launches() == launches
+    ms = E.advance_timed(3)
+    assert list(ms) == launches.split("+") and all(t > 0.0 for t in ms.values()), ms
+    E.close()
