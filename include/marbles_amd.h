@@ -508,6 +508,11 @@ int mrb_population_ptr(const mrb_level *lvl, int lattice, void **dev_ptr, int64_
  * box's scale and was clamped (the per-box scale leaves a factor 16 of
  * headroom; 0 for the other storages).  No reference counterpart. */
 int mrb_storage_saturations(const mrb_level *lvl, int64_t *count);
+/* The steps whose blocks wait for each other (k_step, the z-sweeps) bound
+ * their waits: number of waits since the level was created that ran out, each
+ * of which left NaN in its cells (0 unless such a step failed; 0 for the other
+ * kernels).  Synchronous.  No reference counterpart. */
+int mrb_step_faults(const mrb_level *lvl, int64_t *count);
 /* The rest-state values subtracted by the reduced-precision storages, per
  * direction (zero for FP64), for callers that read the raw buffers of
  * mrb_population_ptr.  No reference counterpart. */

@@ -124,6 +124,7 @@ SIGNATURES = {
     "mrb_hot_kernel_launches": (c_char_p, [c_void_p]),
     "mrb_population_ptr": (c_int, [c_void_p, c_int, POINTER(c_void_p), POINTER(c_int64)]),
     "mrb_storage_saturations": (c_int, [c_void_p, POINTER(c_int64)]),
+    "mrb_step_faults": (c_int, [c_void_p, POINTER(c_int64)]),
     "mrb_storage_shift": (c_int, [c_void_p, c_int, POINTER(c_double)]),
     "mrb_macro_fields": (c_int, [c_void_p, c_void_p, c_void_p]),
     "mrb_vorticity": (c_int, [c_void_p, c_void_p, c_void_p]),

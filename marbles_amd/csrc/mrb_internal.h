@@ -236,7 +236,7 @@ struct mrb_level {
     int32_t *d_isf = nullptr;         // is_fluid, 2 comps
     uint32_t *d_mask = nullptr;       // compact: stream mask per cell
     double *d_md = nullptr;           // FAB: macrodata, 19 comps
-    double *d_dq = nullptr;           // FAB: dQ, 3 comps
+    double *d_dq = nullptr;           // fab: Q_corr, 3 comps
     double *d_q = nullptr;            // compact: Q_corr, 3 comps
     double *d_red = nullptr;          // reduction partials
     double *d_small = nullptr;        // [fshift | gshift | init values | inlet f | inlet g] (6*NQ)
@@ -294,7 +294,7 @@ struct mrb_level {
     int hot_h32 = -1;
     // single-pass z-sweep on 64-cell blocks (k_sweep_x64, compact FP64
     // levels): ring of kSweepRingPlanes planes of Q_y, per-block count of
-    // published planes; count of waits that gave up (both z-sweeps)
+    // published planes; count of waits that gave up (both z-sweeps, k_step)
     double *d_sweep_q = nullptr;
     double *d_sweep_qx = nullptr;  // Q_x of the end cells of 64-cell blocks (k_sweep_x64)
     uint32_t *d_sweep_flags = nullptr;

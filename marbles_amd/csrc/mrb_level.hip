@@ -1271,11 +1271,13 @@ int mrb_level_create(const mrb_level_desc *desc, mrb_level **out)
         MRB_HIP(hipMemset(L->d_mask, 0, sizeof(uint32_t) * T));
         MRB_HIP(hipMalloc(&L->d_q, sizeof(double) * 3 * T));
         MRB_HIP(hipMemset(L->d_q, 0, sizeof(double) * 3 * T));
-        const size_t ntiles = size_t(tiles_per_plane(L->ncell[0], L->ncell[1], 256)) * size_t(L->ncell[2]);
-        MRB_HIP(hipMalloc(&L->d_step_counter, sizeof(unsigned long long)));
-        MRB_HIP(hipMemset(L->d_step_counter, 0, sizeof(unsigned long long)));
-        MRB_HIP(hipMalloc(&L->d_step_flags, sizeof(uint32_t) * ntiles));
-        MRB_HIP(hipMemset(L->d_step_flags, 0, sizeof(uint32_t) * ntiles));
+        if (L->storage == MRB_STORAGE_F64) {
+            const size_t ntiles = size_t(tiles_per_plane(L->ncell[0], L->ncell[1], 256)) * size_t(L->ncell[2]);
+            MRB_HIP(hipMalloc(&L->d_step_counter, sizeof(unsigned long long)));
+            MRB_HIP(hipMemset(L->d_step_counter, 0, sizeof(unsigned long long)));
+            MRB_HIP(hipMalloc(&L->d_step_flags, sizeof(uint32_t) * ntiles));
+            MRB_HIP(hipMemset(L->d_step_flags, 0, sizeof(uint32_t) * ntiles));
+        }
         if (L->storage == MRB_STORAGE_F64 || L->storage == MRB_STORAGE_F32_SHIFTED) {
             const size_t plane = size_t(L->ncell[0]) * size_t(L->ncell[1]);
             const size_t nblk = size_t((L->ncell[0] + 63) / 64) * size_t(L->ncell[1]);
@@ -2300,6 +2302,18 @@ int mrb_storage_saturations(const mrb_level *L, int64_t *count)
     uint32_t v = 0;
     MRB_HIP(hipDeviceSynchronize());
     MRB_HIP(hipMemcpy(&v, L->d_ovf16, sizeof(v), hipMemcpyDeviceToHost));
+    *count = v;
+    return MRB_OK;
+}
+
+int mrb_step_faults(const mrb_level *L, int64_t *count)
+{
+    if (!L || !count) return set_error(MRB_E_ARG, "null argument");
+    *count = 0;
+    if (!L->d_sweep_fault) return MRB_OK;
+    uint32_t v = 0;
+    MRB_HIP(hipDeviceSynchronize());
+    MRB_HIP(hipMemcpy(&v, L->d_sweep_fault, sizeof(v), hipMemcpyDeviceToHost));
     *count = v;
     return MRB_OK;
 }

@@ -29,13 +29,15 @@
 // those have lower list positions, so they were taken before by blocks that
 // are running, and a pass-1 tile waits for nothing.  Every wait therefore
 // ends, however many blocks the GPU holds and whatever else it runs.  (The
-// waits are bounded all the same; past the limit the tile writes NaN.)
+// waits are bounded all the same; past the limit the tile counts a fault, which
+// mrb_step_faults reports, and writes NaN.)
 //
 // Q_corr crosses XCDs, whose L2s are not coherent: it is written and read by
 // agent-scope accesses, and a tile's flag (the launch's epoch) is stored
 // after the tile's Q_corr writes have completed.  Q_x only leaves the block
-// for the tile's two end cells.  The last block to finish resets the list and
-// advances the epoch, so a captured launch can be replayed.
+// for the tile's two end cells.  The block that takes the launch's last entry
+// resets the list and advances the epoch, so a captured launch can be replayed;
+// the blocks still at work keep the epoch they took with their entry.
 #include "compact_cell.h"
 
 namespace mrb {
@@ -89,6 +91,7 @@ struct ListArgs {
     uint32_t wrow;    // tiles a row spans: a tile's y neighbours lie within -+ wrow tiles
     unsigned long long *counter;  // launches so far (high half), list entries taken (low half)
     uint32_t *flags;              // per tile: launch whose Q_corr it holds
+    uint32_t *fault;              // waits that ran out
 };
 
 __device__ __forceinline__ uint32_t load_agent_u32(const uint32_t *p)
@@ -218,6 +221,7 @@ __device__ __forceinline__ void pass2_tile(
         for (uint32_t it = 0; !__syncthreads_and(seen == epoch); ++it) {
             if (it > kStepSpinLimit) {
                 poisoned = true;
+                if (tid == 0) atomicAdd(S.fault, 1u);
                 break;
             }
             __builtin_amdgcn_s_sleep(2);
@@ -385,7 +389,7 @@ int launch(mrb_level *L, hipStream_t s, hipEvent_t *ev)
         if (one_launch(L)) {
             const uint32_t lag = std::min(ntiles, tpp + 1u + kListAhead);
             const ListArgs S{ntiles, lag, uint32_t(A.nx + kStepTile - 1) / kStepTile, L->d_step_counter,
-                             L->d_step_flags};
+                             L->d_step_flags, L->d_sweep_fault};
             k_step<BCX><<<2u * ntiles, kStepTile, 0, s>>>(f, fo, L->d_mask, L->d_q, A, L->bcdev, sh, L->cp, G, S);
             MRB_HIP(hipGetLastError());
             if (ev) MRB_HIP(hipEventRecord(ev[1], s));

@@ -327,6 +327,12 @@ class Level:
         check(self.lib.mrb_storage_saturations(self.h, ctypes.byref(n)))
         return int(n.value)
 
+    def step_faults(self) -> int:
+        """Bounded waits between blocks of a step that ran out so far (each left NaN)."""
+        n = ctypes.c_int64()
+        check(self.lib.mrb_step_faults(self.h, ctypes.byref(n)))
+        return int(n.value)
+
     def shift(self, which: str) -> np.ndarray:
         """Rest-state values subtracted by the reduced-precision storages."""
         out = (c_double * NQ)()

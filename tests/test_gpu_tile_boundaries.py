@@ -115,3 +115,15 @@ def test_timed_steps_name_the_kernels_that_run(engine, storage, shape, variant, 
     ms = E.advance_timed(3)
     assert list(ms) == launches.split("+") and all(t > 0.0 for t in ms.values()), ms
     E.close()
+
+
+@pytest.mark.parametrize("variant", [TILES, "k_sweep", "k_sweep_x64"])
+def test_steps_that_wait_between_blocks_report_no_fault(engine, variant):
+    """k_step and the z-sweeps count the bounded waits that ran out; the count
+    starts at zero and a step that went well leaves it there."""
+    E = configs.build_level(CASES["walls"]((131, 47, 45)), layout="compact")
+    assert E.step_faults() == 0
+    E.set_hot_kernel(variant)
+    E.advance(4)
+    assert E.step_faults() == 0 and np.isfinite(E.valid("f")).all()
+    E.close()
