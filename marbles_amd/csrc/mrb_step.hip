@@ -17,7 +17,7 @@
 // memory-side cache; its loads are non-temporal, since nothing reads the
 // values again.  256^3: 4.30 -> 3.24 ms per step; 301x150x131: 1.95 ->
 // 1.19 ms.  The same traffic through the fabric (22.6 GB) then moves at 7 TB/s,
-// which is what bounds it: a third fewer instructions changed nothing.
+// which is what bounds it: 24 % fewer vector instructions changed nothing.
 // Shifted FP32 storage stays on two launches: pass 2 holds twice the
 // registers of pass 1, so in one kernel pass 1 runs at half its occupancy,
 // and with half the bytes per wave that costs more than the cache saves
@@ -46,10 +46,12 @@ namespace {
 constexpr int kStepTile = 256;
 // FP32 storage: 128-cell tiles (320^3: 4.46 ms against 4.56 with 256)
 constexpr int kF32Tile = 128;
-// k_step takes FP64 levels of at least this many cells: below, launch latency
-// and not memory bounds the step and the work list's counter and flags only
-// add to it (24^3: 14.8 us per step against 12.0 with the passes apart;
-// 660x123x4: 88.7 against 90.6)
+// k_step takes FP64 levels of at least this many cells: below, both passes'
+// populations stay in the memory-side cache anyway (2^18 cells are 113 MB) and
+// the work list's counter and flags only add to the step.  Periodic boxes, us
+// per step in one launch / with the passes apart: 24^3 14.4 / 12.4, 40^3 25.9 /
+// 18.1, 56^3 52.4 / 43.8, 64^3 62.3 / 62.8, 72^3 91.9 / 91.8, 80^3 118 / 126,
+// 96^3 188 / 212, 128^3 414 / 523; thin ones cross later (660x123x4 83.5 / 80.8).
 constexpr int64_t kListCells = 1 << 18;
 // pass-1 tiles ahead of pass 2 besides a plane: the blocks 256 CUs hold at
 // two each, so that the tiles waited for are usually done (256^3: 3.29 ms with
