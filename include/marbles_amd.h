@@ -187,7 +187,7 @@ int mrb_collide(mrb_level *lvl, void *stream);
  * Steps of one level are ordered by the caller (one stream, or events):
  * besides the A/B buffers they share the level's Q-correction array and,
  * for the single-pass sweeps, its ring of published planes and its launch
- * count. */
+ * count, for the one-launch step (k_step) its work list. */
 int mrb_stream_collide(mrb_level *lvl, void *stream);
 /* nsteps fused steps. */
 int mrb_advance(mrb_level *lvl, int nsteps, void *stream);

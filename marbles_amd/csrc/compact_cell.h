@@ -666,7 +666,9 @@ __device__ __forceinline__ void pull_finish(
             // one after the other, each under its lanes' own branch, the
             // waves next to the inlet (two in five on 160-cell rows) waited
             // for nine of them in turn.  A ghost beyond several faces belongs
-            // to the last of x, y, z (BCFill's loop order).
+            // to the last of x, y, z (BCFill's loop order); mrb_set_bc refuses
+            // an OUTFLOW face on an axis after the inlet's, which would copy
+            // another ghost's value here.
             static_for<(BCX & kBcxProfileX) != 0 ? 1 : 6>([&](auto fc) {
                 constexpr int face = decltype(fc)::value, d = face % 3, c = face < 3 ? 1 : -1;
                 constexpr int d1 = d == 0 ? 1 : 0, d2 = d == 2 ? 1 : 2;

@@ -361,7 +361,8 @@ __global__ void __launch_bounds__(TILE, 2) k_collide_tile(
                                      TileCell::of<TILE>(blockIdx.x, A, G), ListArgs{}, 0u);
 }
 // scaled FP16 storage with FP32 arithmetic, held to 128 registers: four
-// waves per SIMD
+// waves per SIMD (with a profile inlet one value spills: 160x80x80 duct 138 us
+// per step against 214 on row blocks without the bound)
 template <class T, int BCX, int ARITH, int TILE>
 __global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) k_collide_tile_w4(
     const T *__restrict__ f, T *__restrict__ fo, const uint32_t *__restrict__ mask, double *__restrict__ Q,

@@ -53,7 +53,7 @@ def test_quiescent_neighbour_boxes_do_not_saturate(engine):
 
 def test_fp32_arithmetic_variant_survives_a_pressure_face(engine):
     """An FP16 level set to the 256x1-block FP32-arithmetic collide that
-    then gets a PRESSURE face steps on the FP64-arithmetic 256x1 variant,
+    then gets a PRESSURE face steps on the FP64-arithmetic tile variant,
     and returns to its own when the faces change back."""
     cfg = configs.pressure_case("walled", (24, 16, 32))
     E = configs.build_level(cfg, layout="compact", storage="f16s")

@@ -262,7 +262,7 @@ def test_f32_shifted_storage_tracks_f64(oracle, engine, case):
 @pytest.mark.parametrize("case", ["tg_tau1.0", "channel_T0.2", "channel_profile"])
 def test_f32_shifted_with_fp32_arithmetic_tracks_f64(engine, case):
     """Shifted FP32 storage with the FP32-arithmetic collide in deviation
-    form (k_collide_f32, 64x2 and 256x1 blocks, bit-identical to each
+    form (k_collide_f32 on 64x2 blocks and the tile step, bit-identical to each
     other): after 100 steps velocity and density within 1e-6 of the FP64
     run (measured 0.99e-7, 4.2e-7 and 1.9e-7 in velocity with the momentum
     residual of the FP32 equilibria returned to the axis pairs; 1.2e-6 and
@@ -468,8 +468,8 @@ def test_f16_storage_with_fp32_arithmetic_tracks_f64(oracle, engine, case):
 
 @pytest.mark.parametrize("case", ["channel", "odd", "channel_profile"])
 def test_fp32_arithmetic_collide_block_shapes_bitwise(engine, case):
-    """The FP32-arithmetic FP16 collide on 256x1-cell blocks equals the
-    64x4 one bit for bit (same operations per cell)."""
+    """The FP32-arithmetic FP16 collide on 256x1-cell row blocks equals the
+    default tile step bit for bit (same operations per cell)."""
     if case == "channel":
         cfg = configs.channel_sphere((48, 24, 24), radius=5.0, center=(16.0, 12.0, 12.0))
     elif case == "odd":
@@ -727,7 +727,7 @@ def test_ic_plugin_workloads_match_oracle(oracle, engine, case, layout):
 @pytest.mark.parametrize("storage", ["f64", "f32s", "f16s"])
 @pytest.mark.parametrize("case", ["channel", "odd", "channel_profile", "pressure_walled", "outlet", "slip"])
 def test_step_variants_equal_two_pass_bitwise(engine, case, storage):
-    """The other block shapes of the two passes (64x8, 64x2, 128x2, 256x1),
+    """The other block shapes of the two passes (64x8, 64x2, 128x2, tiles),
     k_onepass, which recomputes the neighbours' Q_corr from their pulls
     instead of reading pass 1's array, and the single-pass z-sweeps k_sweep
     (FP64 and FP32 storage) and k_sweep_x64 (FP64), which pass Q_corr
